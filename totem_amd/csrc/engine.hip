@@ -378,36 +378,82 @@ struct PotDev {
   int np = 0, S = 0;
   const double *kx1 = nullptr, *ky1 = nullptr, *s2 = nullptr, *aper = nullptr, *corr = nullptr;
   const PotClass* classes = nullptr;
+  int n_classes = 0;
+  bool absorptive = false;  // some class has an absorptive part
   const double *tx = nullptr, *ty = nullptr, *wt = nullptr;
   const PotSeg* segs = nullptr;
   std::vector<long> term_off, seg_off;  // host, [S + 1]
-  size_t max_terms = 0;
   double sigma = 0.0, parameter = 0.0;
   bool sym = false;  // paired frequencies: a quarter of the tiles (hermitian_pairs)
 };
 
-// Per slice: phase tables, reciprocal-space accumulation, unnormalised inverse FFT
-// with exp(i sigma/1000 V) fused into its column pass (or V copied out when asked).
-void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, hipStream_t st, DevBuf& dex,
-                   DevBuf& dey) {
+// Scratch of potential builds: phase tables, form factors, slice entries.
+struct PotScratch {
+  DevBuf ex, ey, ff, slices;
+  size_t bytes() const { return ex.bytes + ey.bytes + ff.bytes; }
+  void release() {
+    ex.release();
+    ey.release();
+    ff.release();
+  }
+};
+
+// Phase tables of a chunk of slices (ex and ey together) up to this size, so that the
+// accumulation reads them from the memory-side cache; a slice above it is a chunk of
+// its own.
+constexpr size_t kPhaseChunkBytes = 96ull << 20;
+// Form factors are tabulated up to this size.
+constexpr size_t kFormTableBytes = 512ull << 20;
+
+// The stack in chunks of slices, four launches per chunk: phase tables, reciprocal-space
+// accumulation, unnormalised inverse FFT (two passes) with exp(i sigma/1000 V) fused into
+// its column pass (or V copied out when asked).  One slice alone fills the chip only at
+// the largest grids (a 256^2 slice has 25 tiles) and its launches are as long as their
+// start-up: 20 slices of 256^2 took 20 x 23 us of kernels, in one chunk 85 us.
+// Form factors are tabulated when each class is used by two slices or more
+// on average; with as many classes as runs of terms the table would only move them
+// through memory.
+void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, hipStream_t st, PotScratch& sc) {
   const int np = p.np, S = p.S;
   const size_t np2 = (size_t)np * np;
-  reserve(dex, std::max<size_t>(p.max_terms, 1) * np * sizeof(float2));
-  reserve(dey, std::max<size_t>(p.max_terms, 1) * np * sizeof(float2));
+  const size_t term_bytes = 2 * (size_t)phase_columns(np, p.sym) * sizeof(float2);
+  const long per_chunk = std::max<long>(1, (long)(kPhaseChunkBytes / term_bytes));
+  std::vector<PotSlice> slices(S);
+  std::vector<int> chunks = {0};  // chunk boundaries
+  long most = 1;
+  for (int s = 0; s < S; ++s) {
+    slices[s] = {(int)p.term_off[s], (int)p.seg_off[s], (int)(p.seg_off[s + 1] - p.seg_off[s])};
+    if (s > chunks.back() && p.term_off[s + 1] - p.term_off[chunks.back()] > per_chunk) chunks.push_back(s);
+    most = std::max(most, p.term_off[s + 1] - p.term_off[chunks.back()]);
+  }
+  chunks.push_back(S);
+  reserve(sc.ex, most * (term_bytes / 2));
+  reserve(sc.ey, most * (term_bytes / 2));
+  upload(sc.slices, slices, st);
+  const size_t ff_bytes = (size_t)p.n_classes * np2 * sizeof(double) * (p.absorptive ? 2 : 1);
+  double *ff_re = nullptr, *ff_im = nullptr;
+  if (p.seg_off[S] >= 2L * p.n_classes && ff_bytes > 0 && ff_bytes <= kFormTableBytes) {
+    reserve(sc.ff, ff_bytes);
+    ff_re = sc.ff.as<double>();
+    if (p.absorptive) ff_im = ff_re + (size_t)p.n_classes * np2;
+    form_table(st, p.classes, p.n_classes, p.s2, p.corr, np, ff_re, ff_im);
+  }
   tw_table(np);
   const float sig = (float)(p.sigma / 1000.0);
   const bool want_v = v_re && v_im;
   std::vector<float2> hv;
   if (want_v) hv.resize(np2);
-  for (int s = 0; s < S; ++s) {
-    const int nt = (int)(p.term_off[s + 1] - p.term_off[s]);
-    float2* ts = t_dev + (size_t)s * np2;
-    phase_tables(st, p.tx + p.term_off[s], p.ty + p.term_off[s], p.wt + p.term_off[s], nt, p.kx1, p.ky1, np, p.sym,
-                 dex.as<float2>(), dey.as<float2>());
-    accumulate(st, dex.as<float2>(), dey.as<float2>(), p.segs + p.seg_off[s],
-               (int)(p.seg_off[s + 1] - p.seg_off[s]), p.classes, p.s2, p.aper, p.corr, p.parameter, np, p.sym, ts);
-    if (want_v) {
-      fft2d(np, st, ts, ts, 1, +1, 0, 0.f);
+  for (size_t c = 0; c + 1 < chunks.size(); ++c) {
+    const int s0 = chunks[c], cnt = chunks[c + 1] - s0;
+    const long t0 = p.term_off[s0];
+    float2* tc = t_dev + (size_t)s0 * np2;
+    phase_tables(st, p.tx + t0, p.ty + t0, p.wt + t0, (int)(p.term_off[s0 + cnt] - t0), p.kx1, p.ky1, np, p.sym,
+                 sc.ex.as<float2>(), sc.ey.as<float2>());
+    accumulate(st, sc.ex.as<float2>(), sc.ey.as<float2>(), sc.slices.as<PotSlice>() + s0, cnt, (int)t0, p.segs,
+               p.classes, ff_re, ff_im, p.s2, p.aper, p.corr, p.parameter, np, p.sym, tc);
+    fft2d(np, st, tc, tc, cnt, +1, want_v ? 0 : 1, want_v ? 0.f : sig);
+    for (int s = s0; want_v && s < s0 + cnt; ++s) {
+      float2* ts = t_dev + (size_t)s * np2;
       HIP_OK(hipMemcpyAsync(hv.data(), ts, np2 * sizeof(float2), hipMemcpyDeviceToHost, st));
       HIP_OK(hipStreamSynchronize(st));
       for (size_t i = 0; i < np2; ++i) {
@@ -417,21 +463,18 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
         hv[i] = make_float2(amp * std::cos(sig * hv[i].x), amp * std::sin(sig * hv[i].x));
       }
       HIP_OK(hipMemcpyAsync(ts, hv.data(), np2 * sizeof(float2), hipMemcpyHostToDevice, st));
-    } else {
-      fft2d(np, st, ts, ts, 1, +1, 1, sig);
     }
     HIP_OK(hipGetLastError());
   }
+  HIP_OK(hipStreamSynchronize(st));
 }
 
 // Flattens a plan's terms slice by slice, stably grouped by class within a slice.
 static void flatten_plan(PotentialPlan& P, std::vector<double>& tx, std::vector<double>& ty, std::vector<double>& wt,
-                         std::vector<PotSeg>& segs, std::vector<long>& term_off, std::vector<long>& seg_off,
-                         size_t& max_terms) {
+                         std::vector<PotSeg>& segs, std::vector<long>& term_off, std::vector<long>& seg_off) {
   const int S = P.S;
   term_off.assign(S + 1, 0);
   seg_off.assign(S + 1, 0);
-  max_terms = 0;
   for (int s = 0; s < S; ++s) {
     auto& v = P.slices[s];
     std::stable_sort(v.begin(), v.end(), [](const Term& a, const Term& b) { return a.cls < b.cls; });
@@ -444,12 +487,11 @@ static void flatten_plan(PotentialPlan& P, std::vector<double>& tx, std::vector<
     }
     term_off[s + 1] = (long)tx.size();
     seg_off[s + 1] = (long)segs.size();
-    max_terms = std::max(max_terms, v.size());
   }
 }
 
-// Phase-table scratch (terms of the largest slice x np x 16 bytes) above this
-// size is released after the build instead of kept for the next one.
+// Builder scratch (phase tables and form factors) above this size is released after
+// the build instead of kept for the next one.
 constexpr size_t kKeepBuilderScratch = 256ull << 20;
 
 static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev, double* v_re, double* v_im,
@@ -459,11 +501,12 @@ static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev
   std::vector<double> tx, ty, wt;
   std::vector<PotSeg> segs;
   PotDev pd;
-  flatten_plan(P, tx, ty, wt, segs, pd.term_off, pd.seg_off, pd.max_terms);
+  flatten_plan(P, tx, ty, wt, segs, pd.term_off, pd.seg_off);
   // per-device builder scratch, one build at a time per device
   struct Scratch {
     std::mutex mu;
-    DevBuf dtx, dty, dwt, dsegs, dcls, dkx, dky, ds2, dap, dcorr, dex, dey;
+    DevBuf dtx, dty, dwt, dsegs, dcls, dkx, dky, ds2, dap, dcorr;
+    PotScratch pot;
   };
   static std::mutex scratch_mu;
   static std::map<int, std::unique_ptr<Scratch>> scratch;
@@ -501,6 +544,8 @@ static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev
   pd.aper = sc->dap.as<double>();
   pd.corr = sc->dcorr.as<double>();
   pd.classes = sc->dcls.as<PotClass>();
+  pd.n_classes = (int)P.classes.size();
+  for (const PotClass& k : P.classes) pd.absorptive = pd.absorptive || k.has_abs;
   pd.tx = sc->dtx.as<double>();
   pd.ty = sc->dty.as<double>();
   pd.wt = sc->dwt.as<double>();
@@ -508,14 +553,8 @@ static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev
   pd.sigma = d.sigma;
   pd.parameter = d.parameter;
   pd.sym = hermitian_pairs(P.kx1.data(), P.ky1.data(), P.np);
-  potential_run(pd, t_dev, v_re, v_im, st, sc->dex, sc->dey);
-  HIP_OK(hipStreamSynchronize(st));
-  // the phase tables grow with the terms of the largest slice; a large set is not
-  // kept for the rest of the process
-  if (sc->dex.bytes + sc->dey.bytes > kKeepBuilderScratch) {
-    sc->dex.release();
-    sc->dey.release();
-  }
+  potential_run(pd, t_dev, v_re, v_im, st, sc->pot);
+  if (sc->pot.bytes() > kKeepBuilderScratch) sc->pot.release();
 }
 
 // ------------------------------------------------------- specimen on the device
@@ -538,7 +577,9 @@ struct totem_specimen {
   size_t sort_bytes = 0;
   totem::DevBuf xyz, rms, pos, faces, term_atom, term_cls, term_w, term_mode, sub_base, keys, keys2, vals, vals2,
       wslot, counts, sort_tmp;
-  totem::DevBuf tx, ty, wt, segs, classes, kx, ky, s2, aper, corr, ex, ey;
+  totem::DevBuf tx, ty, wt, segs, classes, kx, ky, s2, aper, corr;
+  totem::PotScratch pot;
+  bool absorptive = false;
   std::vector<int> h_counts;
   std::vector<totem::PotSeg> h_segs;
 };
@@ -630,6 +671,7 @@ static totem_specimen* specimen_create_impl(const totem_specimen_desc& d) {
   sp->sigma = d.pot.sigma;
   sp->parameter = d.pot.parameter;
   sp->has_rms = d.rms != nullptr;
+  for (const PotClass& k : classes) sp->absorptive = sp->absorptive || k.has_abs;
   sp->sym = hermitian_pairs(P.kx1.data(), P.ky1.data(), np);
   while ((1L << sp->bits) <= (long)S * Ct) ++sp->bits;
   hipStream_t st = lib_stream();
@@ -723,7 +765,6 @@ static void specimen_transmission_impl(totem_specimen& sp, uint64_t seed, int co
     total += in_slice;
     pd.term_off[s + 1] = total;
     pd.seg_off[s + 1] = (long)sp.h_segs.size();
-    pd.max_terms = std::max<size_t>(pd.max_terms, (size_t)in_slice);
   }
   require(total <= n2, "specimen: internal count mismatch");
   if (!sp.h_segs.empty())
@@ -740,6 +781,8 @@ static void specimen_transmission_impl(totem_specimen& sp, uint64_t seed, int co
   pd.aper = sp.aper.as<double>();
   pd.corr = sp.corr.as<double>();
   pd.classes = sp.classes.as<PotClass>();
+  pd.n_classes = C;
+  pd.absorptive = sp.absorptive;
   pd.tx = sp.tx.as<double>();
   pd.ty = sp.ty.as<double>();
   pd.wt = sp.wt.as<double>();
@@ -747,8 +790,7 @@ static void specimen_transmission_impl(totem_specimen& sp, uint64_t seed, int co
   pd.sigma = sp.sigma;
   pd.parameter = sp.parameter;
   pd.sym = sp.sym;
-  potential_run(pd, t_dev, nullptr, nullptr, st, sp.ex, sp.ey);
-  HIP_OK(hipStreamSynchronize(st));
+  potential_run(pd, t_dev, nullptr, nullptr, st, sp.pot);
 }
 
 // ---------------------------------------------------------------- STEM propagation

@@ -76,4 +76,10 @@ struct PotSeg {
   int begin, end;   // term range relative to the slice's first term
 };
 
+// One slice of a potential build: its first term and its runs of terms.
+struct PotSlice {
+  int term;         // first term in the build's term arrays
+  int seg, n_seg;   // its PotSeg entries
+};
+
 }  // namespace totem

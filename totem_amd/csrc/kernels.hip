@@ -4,8 +4,9 @@
 //  * k_pass_cols  -- per slice, along columns: forward column FFT -> x propagator ->
 //                    [annular detectors] -> inverse column FFT   (exit slice: detectors only)
 //  * k_reduce_det -- per finished probe: fixed-order compensated FP64 sum of detector partials
-//  * k_phase / k_accumulate_mfma16 -- projected potential in reciprocal space per slice
-//                    (structure-factor sums on the matrix cores, 16 x 16 pixel tiles)
+//  * k_form_table / k_phase / k_accumulate_mfma32 -- projected potential in reciprocal space,
+//                    several slices per launch (structure-factor sums on the matrix cores, 32 x 32
+//                    pixel tiles)
 //  * k_fft_rows / k_fft_cols -- plain batched 2-D FFT passes (potential IFFT, tests)
 //
 // A full 2-D forward+inverse FFT per slice therefore costs two read+write
@@ -725,14 +726,20 @@ k_fft_cols(const float2* __restrict__ src, float2* __restrict__ dst, int epi, fl
 // ex[j][c] = w_j exp(-2 pi i kx1[c] x_j), ey[j][r] = exp(-2 pi i ky1[r] y_j); the
 // product k.x is formed and reduced modulo 1 in FP64 before the (FP64) sincospi, and
 // the term's weight is applied in FP64 before the rounding to FP32.  Only the first
-// nc entries of each table are formed (the accumulation reads no more).
-__global__ void k_phase(const double* __restrict__ tx, const double* __restrict__ ty,
-                        const double* __restrict__ wt, int n_terms, const double* __restrict__ kx1,
-                        const double* __restrict__ ky1, int np, int nc, float2* __restrict__ ex,
-                        float2* __restrict__ ey) {
+// nc entries of each row are formed and stored (the accumulation reads no more);
+// entries at or beyond np, in the last tile's overhang, are zero.
+__global__ void __launch_bounds__(256) k_phase(const double* __restrict__ tx, const double* __restrict__ ty,
+                                               const double* __restrict__ wt, const double* __restrict__ kx1,
+                                               const double* __restrict__ ky1, int np, int nc,
+                                               float2* __restrict__ ex, float2* __restrict__ ey) {
   const int c = blockIdx.y * blockDim.x + threadIdx.x;
   const int j = blockIdx.x;
-  if (c >= nc || j >= n_terms) return;
+  if (c >= nc) return;
+  const size_t at = (size_t)j * nc + c;
+  if (c >= np) {
+    ex[at] = ey[at] = make_float2(0.f, 0.f);
+    return;
+  }
   double fx = kx1[c] * tx[j];
   fx -= rint(fx);
   double fy = ky1[c] * ty[j];
@@ -741,8 +748,8 @@ __global__ void k_phase(const double* __restrict__ tx, const double* __restrict_
   sincospi(2.0 * fx, &sx, &cx);
   sincospi(2.0 * fy, &sy, &cy);
   const double w = wt[j];
-  ex[(size_t)j * np + c] = make_float2((float)(w * cx), (float)(-w * sx));
-  ey[(size_t)j * np + c] = make_float2((float)cy, (float)-sy);
+  ex[at] = make_float2((float)(w * cx), (float)(-w * sx));
+  ey[at] = make_float2((float)cy, (float)-sy);
 }
 
 // Terms with a zero coefficient are skipped: the one-term classes of erf-weighted
@@ -783,14 +790,28 @@ __device__ __forceinline__ double2 form_factor(const PotClass& k, double s2, con
   return make_double2(re, im);
 }
 
-// One slice: V_k(r,c) = PARAMETER * AperTrue * sum_classes f_cls(k) * sum_{j in cls} w_j ex_j[c] ey_j[r],
+// ff_re[cls][pix] (and ff_im where some class is absorptive): the form factors of
+// every class at every pixel, formed once per build.  A slice's accumulation then reads
+// 8 bytes per class and pixel instead of evaluating up to ten FP64 exponentials there,
+// which every slice of the stack would repeat.
+__global__ void __launch_bounds__(256) k_form_table(const PotClass* __restrict__ classes, const double* __restrict__ s2,
+                                                    const double* __restrict__ corr, size_t np2,
+                                                    double* __restrict__ ff_re, double* __restrict__ ff_im) {
+  const size_t pix = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (pix >= np2) return;
+  const double2 f = form_factor(classes[blockIdx.y], s2[pix], corr, pix, np2);
+  ff_re[blockIdx.y * np2 + pix] = f.x;
+  if (ff_im) ff_im[blockIdx.y * np2 + pix] = f.y;
+}
+
+// Slices of a chunk: V_k(r,c) = PARAMETER * AperTrue * sum_classes f_cls(k) * sum_{j in cls} w_j ex_j[c] ey_j[r],
 // written at the ifftshifted position (the reference's quadrant swap) as complex64.
 //
 // Per class the sum over terms is a complex matrix product, A[r][j] = ey_j[r] times
-// B[j][c] = ex_j[c] (the weight w_j already in ex), on the matrix cores in FP32 (v_mfma_f32_16x16x4f32, four
-// terms per product): lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16], and
-// accumulator element i of lane l is C[4 (l / 16) + i][l % 16].  The four real
-// products are kept apart,
+// B[j][c] = ex_j[c] (the weight w_j already in ex), on the matrix cores in FP32
+// (v_mfma_f32_32x32x2f32, two terms per product): lane l supplies A[l % 32][l / 32] and
+// B[l / 32][l % 32], and accumulator element i of lane l is
+// C[8 (i / 4) + 4 (l / 32) + i % 4][l % 32].  The four real products are kept apart,
 //   P1 = Ar Br,  P2 = Ai Bi,  P3 = Ar Bi,  P4 = Ai Br  (summed over terms),
 // because the weights are real and the grid's frequencies come in pairs
 // (ky[N - r] = -ky[r], kx[N - c] = -kx[c]): then ey_j[N - r] = conj(ey_j[r]) and
@@ -799,113 +820,169 @@ __device__ __forceinline__ double2 form_factor(const PotClass& k, double s2, con
 //   S(r, N - c)     = (P1 + P2) + i (P4 - P3)
 //   S(N - r, c)     = (P1 + P2) + i (P3 - P4)
 //   S(N - r, N - c) = (P1 - P2) - i (P3 + P4).
-// With `sym` set the tiles cover rows and columns [0, N/2 + 16) (the Nyquist row
-// and column, which have no pair, among them) and rows / columns r in
-// [1, N/2 - 16] also write their pair N - r: every pixel is written once.
-// Without it (a grid whose frequencies are not paired) the tiles cover the grid.
-// W waves share a tile, each taking every W-th group of 16 terms of a class; the
-// partial products are summed in LDS and each thread then weights one tile
-// position's pixels by the class's FP64 form factor at each of them.
-#ifndef TOTEM_ACC_MINWAVES
-#define TOTEM_ACC_MINWAVES 1  // minimum waves per SIMD the accumulation is compiled for
+// With `sym` set the tiles cover rows and columns [0, N/2] (r = 0 and N/2 have no pair)
+// and rows / columns in [1, N/2 - 1] also write their pair N - r: every pixel is
+// written once.  Without it (a grid whose frequencies are not paired) the tiles cover
+// the grid.
+// W waves share a 32 x 32 tile, each taking every W-th group of 8 terms of a class; the
+// partial products are summed in LDS, one product per round through two alternating
+// buffers, and each thread then weights two tile positions' pixels by the class's FP64
+// form factor at each of them.  A 32 x 32 tile reads 512 bytes of phases per term for
+// 4096 multiply-adds, half the operand traffic of a 16 x 16 one, and the next group's
+// phases are in flight during the 16 products of the current one.  Bound by the matrix
+// cores and, behind them, the phases from L2 (about 5 TB/s): a 1024^2 slice of 2000
+// terms takes 64 us, of which 31 us are its products at the FP32 matrix rate (16 x 16
+// tiles with the form factors evaluated in the kernel: 100 us).  Four waves per tile
+// (216 VGPRs, two tiles per CU, so one's reduction overlaps the other's products)
+// measure as eight at 128 VGPRs do, which spill; groups of 8 terms are 5% faster than
+// groups of 4.
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+#ifndef TOTEM_ACC_STEPS
+#define TOTEM_ACC_STEPS 4
 #endif
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-template <int W>
+#ifndef TOTEM_ACC_MINWAVES
+#define TOTEM_ACC_MINWAVES 2
+#endif
+enum FormMode : int { kFormEval, kFormRe, kFormComplex };
+template <int W, int FORM>
 __global__ void __launch_bounds__(64 * W, TOTEM_ACC_MINWAVES)
-k_accumulate_mfma16(const float2* __restrict__ ex, const float2* __restrict__ ey, const PotSeg* __restrict__ segs, int n_segs, const PotClass* __restrict__ classes,
-                    const double* __restrict__ s2, const double* __restrict__ aper_true,
-                    const double* __restrict__ corr, double parameter, int np, int sym,
-                    float2* __restrict__ vshift) {
-  constexpr int NT = 64 * W, NO = 1024 / NT;  // threads; output pixels per thread
-  static_assert(NO * NT == 1024, "four pixels per tile position");
-  __shared__ float red[W * 4 * 4 * 64];      // [wave][product][element][lane]
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int dt = sym ? np / 32 + 1 : np / 16;
-  const int tr = blockIdx.x / dt, tc = blockIdx.x - tr * dt;
-  const int r0 = tr * 16, c0 = tc * 16;
-  const int li = lane & 15, lk = lane >> 4;
+k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey, const PotSlice* __restrict__ slices,
+                    int term_base, const PotSeg* __restrict__ segs, const PotClass* __restrict__ classes,
+                    const double* __restrict__ ff_re, const double* __restrict__ ff_im, const double* __restrict__ s2,
+                    const double* __restrict__ aper_true, const double* __restrict__ corr, double parameter, int np,
+                    int nc, int sym, float2* __restrict__ vshift) {
+  constexpr int U = TOTEM_ACC_STEPS, GT = 2 * U;  // matrix steps, terms per group
+  constexpr int NT = 64 * W, NP = 1024 / NT, NO = 4 * NP;  // threads; positions and pixels per thread
+  static_assert(NP * NT == 1024, "one or more positions per thread");
+  __shared__ float red[2][W * 1024];  // [buffer][wave][element][lane]
+  static_assert(sizeof(red) <= kLdsLimit, "accumulation LDS above 64 KiB");
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int dt = nc / 32, tiles = dt * dt;
+  const int sl = blockIdx.x / tiles, tile = blockIdx.x - sl * tiles;
+  const int tr = tile / dt, tc = tile - tr * dt;
+  const int r0 = tr * 32, c0 = tc * 32;
+  const PotSlice ps = slices[sl];
   const size_t np2 = (size_t)np * np;
-  // this thread's tile position, its LDS source (lane, element) and output pixels
-  const int pos = threadIdx.x & 255;
-  const int pr = pos >> 4, pcl = pos & 15;
-  const int src = (pr >> 2) * 16 + pcl + 64 * (pr & 3);  // source lane + 64 * accumulator element
-  const int r = r0 + pr, c = c0 + pcl;
-  const int pair_hi = np / 2 - 16;
-  bool valid[NO];
-  bool cj_r[NO], cj_c[NO];
-  size_t pix[NO];
-  double s2v[NO], vr[NO], vi[NO];
+  const int half = np / 2;
+  // this thread's positions (accumulator element and lane at which they are summed) and pixels
+  int pix[NO];  // -1: no such pixel
+  double s2v[FORM == kFormEval ? NO : 1], vr[NO], vi[NO];
 #pragma unroll
-  for (int o = 0; o < NO; ++o) {
-    const int quad = (threadIdx.x >> 8) + (NT >> 8) * o;  // bit 0: column pair, bit 1: row pair
-    cj_c[o] = quad & 1;
-    cj_r[o] = (quad >> 1) & 1;
-    valid[o] = (!cj_r[o] || (sym && r >= 1 && r <= pair_hi)) && (!cj_c[o] || (sym && c >= 1 && c <= pair_hi));
-    const int R = cj_r[o] ? np - r : r, C = cj_c[o] ? np - c : c;
-    pix[o] = (size_t)R * np + C;
-    s2v[o] = valid[o] ? s2[pix[o]] : 0.0;
-    vr[o] = vi[o] = 0.0;
+  for (int u = 0; u < NP; ++u) {
+    const int pos = threadIdx.x + NT * u, i = pos >> 6, l = pos & 63;
+    const int r = r0 + 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), c = c0 + (l & 31);
+#pragma unroll
+    for (int quad = 0; quad < 4; ++quad) {  // bit 0: column pair, bit 1: row pair
+      const bool cj_c = quad & 1, cj_r = quad >> 1;
+      const int o = 4 * u + quad;
+      const bool ok = sym ? (r <= half && c <= half && (!cj_r || (r >= 1 && r < half)) &&
+                             (!cj_c || (c >= 1 && c < half)))
+                          : quad == 0;
+      pix[o] = ok ? (cj_r ? np - r : r) * np + (cj_c ? np - c : c) : -1;
+      if constexpr (FORM == kFormEval) s2v[o] = ok ? s2[pix[o]] : 0.0;
+      vr[o] = vi[o] = 0.0;
+    }
   }
-  for (int sgi = 0; sgi < n_segs; ++sgi) {
-    const PotSeg sg = segs[sgi];
-    floatx4 p1 = {}, p2 = {}, p3 = {}, p4 = {};
-    for (int j = sg.begin + 16 * wave; j < sg.end; j += 16 * W) {
-      float2 a[4], b[4];
+  // byte offsets of this lane's phases in a group of terms
+  int oa[U], ob[U];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int jj = j + 4 * u + lk;
-        a[u] = b[u] = make_float2(0.f, 0.f);
-        if (jj < sg.end) {
-          a[u] = ey[(size_t)jj * np + r0 + li];
-          b[u] = ex[(size_t)jj * np + c0 + li];
+  for (int u = 0; u < U; ++u) {
+    const int row = (2 * u + (lane >> 5)) * nc;
+    oa[u] = (row + r0 + (lane & 31)) * (int)sizeof(float2);
+    ob[u] = (row + c0 + (lane & 31)) * (int)sizeof(float2);
+  }
+  for (int sgi = ps.seg; sgi < ps.seg + ps.n_seg; ++sgi) {
+    const PotSeg sg = segs[sgi];
+    const int base = ps.term - term_base;
+    floatx16 p1 = {}, p2 = {}, p3 = {}, p4 = {};
+    float2 a[U], b[U], an[U], bn[U];
+    // phases of the group of terms [j, j + GT) (zero beyond the class's last term)
+    auto load = [&](int j, float2* x, float2* y) {
+      const int left = min(max(sg.end - j, 0), GT);
+      const size_t at = (size_t)(base + j) * nc;
+      const auto ra = buf_rsrc(ey + at, (unsigned)(left * nc * (int)sizeof(float2)));
+      const auto rb = buf_rsrc(ex + at, (unsigned)(left * nc * (int)sizeof(float2)));
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        x[u] = bld(ra, oa[u], 0);
+        y[u] = bld(rb, ob[u], 0);
+      }
+    };
+    int j = sg.begin + GT * wave;
+    if (j < sg.end) load(j, a, b);
+    for (; j < sg.end; j += GT * W) {
+      load(j + GT * W, an, bn);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].x, p1, 0, 0, 0);
+        p2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].y, p2, 0, 0, 0);
+        p3 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].y, p3, 0, 0, 0);
+        p4 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].x, p4, 0, 0, 0);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        a[u] = an[u];
+        b[u] = bn[u];
+      }
+    }
+    float q[4][NP];
+    auto reduce = [&](int k, const floatx16& p) {
+      float* const mine = red[k & 1] + wave * 1024 + lane;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mine[64 * i] = p[i];
+      __syncthreads();
+#pragma unroll
+      for (int u = 0; u < NP; ++u) {
+        float t = 0.f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) t += red[k & 1][w * 1024 + threadIdx.x + NT * u];
+        q[k][u] = t;
+      }
+    };
+    reduce(0, p1);
+    reduce(1, p2);
+    double fr[NO], fi[NO];
+    if constexpr (FORM != kFormEval) {
+#pragma unroll
+      for (int o = 0; o < NO; ++o) {
+        const size_t at = sg.cls * np2 + max(pix[o], 0);
+        fr[o] = ff_re[at];
+        if constexpr (FORM == kFormComplex) fi[o] = ff_im[at];
+      }
+    }
+    reduce(2, p3);
+    reduce(3, p4);
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+#pragma unroll
+      for (int quad = 0; quad < 4; ++quad) {
+        const bool cj_c = quad & 1, cj_r = quad >> 1;
+        const int o = 4 * u + quad;
+        if constexpr (FORM == kFormEval) {
+          if (pix[o] < 0) continue;
+          const double2 f = form_factor(classes[sg.cls], s2v[o], corr, pix[o], np2);
+          fr[o] = f.x;
+          fi[o] = f.y;
+        }
+        const double sre = cj_r == cj_c ? (double)(q[0][u] - q[1][u]) : (double)(q[0][u] + q[1][u]);
+        const double sim = (double)(cj_c ? -q[2][u] : q[2][u]) + (double)(cj_r ? -q[3][u] : q[3][u]);
+        if constexpr (FORM == kFormRe) {
+          vr[o] += fr[o] * sre;
+          vi[o] += fr[o] * sim;
+        } else {
+          vr[o] += fr[o] * sre - fi[o] * sim;
+          vi[o] += fr[o] * sim + fi[o] * sre;
         }
       }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        p1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].x, p1, 0, 0, 0);
-        p2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].y, p2, 0, 0, 0);
-        p3 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].y, p3, 0, 0, 0);
-        p4 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].x, p4, 0, 0, 0);
-      }
-    }
-    float* const mine = red + wave * 1024;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      mine[0 * 256 + 64 * i + lane] = p1[i];
-      mine[1 * 256 + 64 * i + lane] = p2[i];
-      mine[2 * 256 + 64 * i + lane] = p3[i];
-      mine[3 * 256 + 64 * i + lane] = p4[i];
-    }
-    __syncthreads();
-    float q1 = 0.f, q2 = 0.f, q3 = 0.f, q4 = 0.f;
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-      const float* o = red + w * 1024 + src;
-      q1 += o[0];
-      q2 += o[256];
-      q3 += o[512];
-      q4 += o[768];
-    }
-    __syncthreads();  // red is rewritten by the next class
-    const PotClass& cls = classes[sg.cls];
-#pragma unroll
-    for (int o = 0; o < NO; ++o) {
-      if (!valid[o]) continue;
-      const double sre = cj_r[o] == cj_c[o] ? (double)(q1 - q2) : (double)(q1 + q2);
-      const double sim = (double)(cj_c[o] ? -q3 : q3) + (double)(cj_r[o] ? -q4 : q4);
-      const double2 f = form_factor(cls, s2v[o], corr, pix[o], np2);
-      vr[o] += f.x * sre - f.y * sim;
-      vi[o] += f.x * sim + f.y * sre;
-    }
   }
-  const int half = np / 2;
+  float2* const out = vshift + sl * np2;
 #pragma unroll
   for (int o = 0; o < NO; ++o) {
-    if (!valid[o]) continue;
-    const int R = (int)(pix[o] / np), C = (int)(pix[o] - (size_t)R * np);
+    if (pix[o] < 0) continue;
+    const int R = pix[o] / np, C = pix[o] - R * np;
     const double scale = parameter * aper_true[pix[o]];
-    const int rs = (R + half) % np, cs = (C + half) % np;
-    vshift[(size_t)rs * np + cs] = make_float2((float)(vr[o] * scale), (float)(vi[o] * scale));
+    const int rs = R < half ? R + half : R - half, cs = C < half ? C + half : C - half;
+    out[(size_t)rs * np + cs] = make_float2((float)(vr[o] * scale), (float)(vi[o] * scale));
   }
 }
 
@@ -1193,36 +1270,52 @@ void fft2d(int n, hipStream_t st, float2* data, float2* dst, int batch, int sign
 }
 
 bool hermitian_pairs(const double* kx1, const double* ky1, int np) {
-  if (np % 32 != 0) return false;
-  for (int r = 1; r <= np / 2 - 16; ++r)
+  if (np % 2 != 0) return false;
+  for (int r = 1; r < np / 2; ++r)
     if (ky1[np - r] != -ky1[r] || kx1[np - r] != -kx1[r]) return false;
   return true;
 }
 
-int phase_columns(int np, bool sym) { return sym ? np / 2 + 16 : np; }
+// whole 32-entry tiles of [0, np/2] (paired frequencies) or of [0, np)
+int phase_columns(int np, bool sym) { return ((sym ? np / 2 + 1 : np) + 31) / 32 * 32; }
 
 void phase_tables(hipStream_t st, const double* tx, const double* ty, const double* wt, int n_terms,
                   const double* kx1, const double* ky1, int np, bool sym, float2* ex, float2* ey) {
   if (n_terms <= 0) return;
   const int nc = phase_columns(np, sym);
-  hipLaunchKernelGGL(k_phase, dim3(n_terms, (nc + 255) / 256), dim3(256), 0, st, tx, ty, wt, n_terms, kx1, ky1, np,
-                     nc, ex, ey);
+  hipLaunchKernelGGL(k_phase, dim3(n_terms, (nc + 255) / 256), dim3(256), 0, st, tx, ty, wt, kx1, ky1, np, nc, ex,
+                     ey);
+}
+
+void form_table(hipStream_t st, const PotClass* classes, int n_classes, const double* s2, const double* corr, int np,
+                double* ff_re, double* ff_im) {
+  const size_t np2 = (size_t)np * np;
+  if (n_classes > 0)
+    hipLaunchKernelGGL(k_form_table, dim3((unsigned)((np2 + 255) / 256), n_classes), dim3(256), 0, st, classes, s2,
+                       corr, np2, ff_re, ff_im);
 }
 
 #ifndef TOTEM_ACC_WAVES
-#define TOTEM_ACC_WAVES 8  // waves sharing one potential tile
+#define TOTEM_ACC_WAVES 4  // waves sharing one potential tile
 #endif
 
-void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSeg* segs, int n_segs,
-                const PotClass* classes, const double* s2, const double* aper_true, const double* corr,
-                double parameter, int np, bool sym, float2* vshift) {
-#define X(S) static_assert(S % 16 == 0, "potential tiles need grid sides that are multiples of 16");
+void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSlice* slices, int n_slices,
+                int term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
+                const double* s2, const double* aper_true, const double* corr, double parameter, int np, bool sym,
+                float2* vshift) {
+#define X(S) static_assert(S % 32 == 0 && S <= 32768, "potential tiles: whole tiles without pairs, 32-bit pixels");
   TOTEM_FOR_SIZES(X)
 #undef X
-  const int dt = sym ? np / 32 + 1 : np / 16;
+  const int nc = phase_columns(np, sym), dt = nc / 32;
   constexpr int W = TOTEM_ACC_WAVES;
-  hipLaunchKernelGGL((k_accumulate_mfma16<W>), dim3((unsigned)(dt * dt)), dim3(64 * W), 0, st, ex, ey, segs, n_segs,
-                     classes, s2, aper_true, corr, parameter, np, sym ? 1 : 0, vshift);
+  const dim3 grid((unsigned)(n_slices * dt * dt));
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * W), 0, st, ex, ey, slices, term_base, segs, classes, ff_re, ff_im, s2,
+                       aper_true, corr, parameter, np, nc, sym ? 1 : 0, vshift);
+  };
+  if (ff_im) launch(k_accumulate_mfma32<W, kFormComplex>);
+  else if (ff_re) launch(k_accumulate_mfma32<W, kFormRe>);
+  else launch(k_accumulate_mfma32<W, kFormEval>);
 }
 
 }  // namespace totem

@@ -58,16 +58,23 @@ void fft2d(int n, hipStream_t st, float2* data, float2* dst, int batch, int sign
 void fill(hipStream_t st, float2* p, long n, float re, float im);
 void fill(hipStream_t st, double* p, long n, double v);
 // True when the grid's frequencies pair up (ky1[np - r] = -ky1[r], kx1[np - c] = -kx1[c]
-// for 1 <= r, c <= np/2 - 16) and np is a multiple of 32: the accumulation then
-// forms a quarter of the tiles and writes each one's mirrored pixels too.
+// for 1 <= r, c < np/2): the accumulation then forms a quarter of the tiles and writes
+// each one's mirrored pixels too.
 bool hermitian_pairs(const double* kx1, const double* ky1, int np);
-// Entries per phase table the accumulation reads (np/2 + 16 with paired frequencies).
+// Entries per term of a phase table (whole tiles; about np/2 with paired frequencies).
 int phase_columns(int np, bool sym);
+// ex, ey [n_terms][phase_columns(np, sym)] of the terms.
 void phase_tables(hipStream_t st, const double* tx, const double* ty, const double* wt, int n_terms,
                   const double* kx1, const double* ky1, int np, bool sym, float2* ex, float2* ey);
-void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSeg* segs, int n_segs,
-                const PotClass* classes, const double* s2, const double* aper_true, const double* corr,
-                double parameter, int np, bool sym, float2* vshift);
+// Form factors of every class at every pixel, ff_re / ff_im [n_classes][np][np] (ff_im may be null).
+void form_table(hipStream_t st, const PotClass* classes, int n_classes, const double* s2, const double* corr, int np,
+                double* ff_re, double* ff_im);
+// V(k) of slices[0, n_slices) into vshift [n_slices][np][np]; the phase tables start at
+// term `term_base`.  ff_re null: form factors are evaluated per slice and pixel.
+void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSlice* slices, int n_slices,
+                int term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
+                const double* s2, const double* aper_true, const double* corr, double parameter, int np, bool sym,
+                float2* vshift);
 
 // Specimen slicing on the device (specimen.hip).
 void displace(hipStream_t st, int n, const double* xyz, const double* rms, uint64_t seed, int config, double lo,
