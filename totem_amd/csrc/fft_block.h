@@ -209,6 +209,69 @@ template <int R, int SIGN> __device__ __forceinline__ void dft(float2* a) {
   else static_assert(R == 2, "unsupported radix");
 }
 
+// ------------------------------------------------ twiddled DFTs (fused form)
+// y_k = sum_n a_n (w W_R^k)^n for R = 2^L, W_R = exp(SIGN 2 pi i / R), in place, natural
+// order: a stage's twiddles w^n and its DFT in one evaluation of the polynomial
+// sum_n a_n z^n at z = w W_R^k.  Even and odd halves give y_k, y_(k + R/2) =
+// E_k +- z_k O_k, so every level is R/2 butterflies (e, o) -> (e + f o, e - f o), each
+// six FMAs: four for e + f o, and 2 e - (e + f o) for the other.  The factors f of a
+// level with m outputs per half are w^(R/2m) W_2m^j, j < m/2, and those times SIGN i:
+// R/2 numbers in all (for R = 16 eight instead of the fifteen w^n), read from a table
+// in which each is rounded from its own FP64 value.  16 points take 192 FP32
+// instructions against 60 (products by w^n) + 184 (DFT).
+
+// (e, o) -> (e + f o, e - f o); ROT: with SIGN i f in the place of f
+template <int SIGN, bool ROT> __device__ __forceinline__ void twiddle_pair(float2& e, float2& o, float2 f) {
+  const float fx = f.x, fy = SIGN < 0 ? f.y : -f.y;  // the table holds SIGN = -1
+  float2 t;
+  if constexpr (!ROT) {
+    t.x = fmaf(-fy, o.y, fmaf(fx, o.x, e.x));
+    t.y = fmaf(fy, o.x, fmaf(fx, o.y, e.y));
+  } else if constexpr (SIGN < 0) {  // -i f o
+    t.x = fmaf(fy, o.x, fmaf(fx, o.y, e.x));
+    t.y = fmaf(fy, o.y, fmaf(-fx, o.x, e.y));
+  } else {  // i f o
+    t.x = fmaf(-fy, o.x, fmaf(-fx, o.y, e.x));
+    t.y = fmaf(-fy, o.y, fmaf(fx, o.x, e.y));
+  }
+  o = make_float2(fmaf(2.f, e.x, -t.x), fmaf(2.f, e.y, -t.y));
+  e = t;
+}
+
+// One level: sub-transforms of M outputs, one per residue n < R / M with its outputs
+// at a[n + (R/M) k], joined in pairs (n, n + R/2M); f: this level's factors.
+template <int R, int M, int SIGN> __device__ __forceinline__ void twiddled_levels(float2* a, const float2* f) {
+  if constexpr (M < R) {
+    constexpr int Q = R / (2 * M), NF = M > 1 ? M / 2 : 1;  // residues after this level, factors
+    float2 out[R];
+#pragma unroll
+    for (int n = 0; n < Q; ++n)
+#pragma unroll
+      for (int k = 0; k < M; ++k) {
+        float2 e = a[n + 2 * Q * k], o = a[n + Q + 2 * Q * k];
+        if (k < NF) twiddle_pair<SIGN, false>(e, o, f[k]);
+        else twiddle_pair<SIGN, true>(e, o, f[k - NF]);
+        out[n + Q * k] = e;
+        out[n + Q * (k + M)] = o;
+      }
+#pragma unroll
+    for (int r = 0; r < R; ++r) a[r] = out[r];
+    twiddled_levels<R, 2 * M, SIGN>(a, f + NF);
+  }
+}
+template <int R, int SIGN> __device__ __forceinline__ void twiddled_dft(float2* a, const float2* f) {
+  twiddled_levels<R, 1, SIGN>(a, f);
+}
+// Factor q < R/2 of the fused form as (power of w, W_R exponent): factors of level M in order.
+constexpr int fused_power(int R, int q, bool rotation) {
+  for (int M = 1; M < R; M *= 2) {
+    const int nf = M > 1 ? M / 2 : 1;
+    if (q < nf) return rotation ? q * (R / (2 * M)) : R / (2 * M);
+    q -= nf;
+  }
+  return 0;
+}
+
 // ------------------------------------------------------------------ Stockham stages
 //
 // Stage with radix R after radices of product P (P = 1 for the first stage):
@@ -219,7 +282,9 @@ template <int R, int SIGN> __device__ __forceinline__ void dft(float2* a) {
 // Twiddles: the plan's table holds, for every stage after the first, the factors
 // exp(-2 pi i q k / (P R)) for q < R and k < P, q-major (pairs of q for even R), so
 // that one load instruction of a wave, whose lanes hold neighbouring k, reads
-// neighbouring entries (16-byte loads for even R).
+// neighbouring entries (16-byte loads for even R).  Plans in fused form (FUSED) run
+// their stages of radix 2, 4, 8 and 16 as twiddled DFTs (above), with the R/2 factors
+// of that form in the table.
 //
 // LDS: with PP (ping-pong) two buffers are used alternately, so one barrier per
 // exchange suffices (the next exchange writes the other buffer, and the one after
@@ -245,7 +310,15 @@ template <bool WAVE> __device__ __forceinline__ void lds_sync() {
 // per transform (elements [0, N/2) first, then [N/2, N)), for lengths whose full
 // exchange buffer would not fit.  A lane reads elements t + T*v, which lie in the
 // lower half exactly for v < E/2; the writes of a round are predicated per element.
-template <int N, int T, int SIGN, class Lay, bool PP, int P, int PING, bool SPLIT, int... RS> struct Stages;
+template <int N, int T, int SIGN, class Lay, bool PP, int P, int PING, bool SPLIT, bool FUSED, int... RS> struct Stages;
+
+// Entries a stage's table of n entries takes: an even number, so that the next stage's
+// 16-byte reads stay aligned.
+__host__ __device__ constexpr int stage_table_len(int n) { return (n + 1) & ~1; }
+// Whether a stage of radix R runs in fused form, and the table entries per k of a stage.
+__host__ __device__ constexpr bool fused_radix(int R) { return R % 2 == 0; }
+template <int R, bool FUSED> constexpr bool fused_stage() { return FUSED && fused_radix(R); }
+template <int R, bool FUSED> constexpr int stage_factors() { return fused_stage<R, FUSED>() ? R / 2 : R; }
 
 // Twiddles of the stage (P, R) for the U butterflies of lane t: block k = b mod P
 // of the stage table, R entries (index u*R + q; entry 0 is 1).  A stage's loads
@@ -256,56 +329,57 @@ template <int N, int T, int SIGN, class Lay, bool PP, int P, int PING, bool SPLI
 #ifndef TOTEM_TW_LATE
 #define TOTEM_TW_LATE 1
 #endif
-template <int T, int P, int R, int U> struct StageTw {
-  static constexpr int NW = (P > 1) ? U * R : 1;
+template <int T, int P, int R, int U, bool FUSED> struct StageTw {
+  static constexpr int F = stage_factors<R, FUSED>();  // entries per butterfly
+  static constexpr int NW = (P > 1) ? U * F : 1;
   float2 w[NW];
   __device__ __forceinline__ void load(const float2* __restrict__ tw, int t) {
     if constexpr (P > 1) {
       // buffer loads: the lane's k in the vector offset, the q part in the scalar
       // offset (no 64-bit address per q)
-      const auto rs = buf_rsrc(tw, (unsigned)(P * R * sizeof(float2)));
+      const auto rs = buf_rsrc(tw, (unsigned)(P * F * sizeof(float2)));
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int k = (t + T * u) % P;
-        if constexpr (R % 2 == 0) {
+        if constexpr (F % 2 == 0) {
 #pragma unroll
-          for (int j = 0; j < R / 2; ++j) {
+          for (int j = 0; j < F / 2; ++j) {
             const float4 v = bld4(rs, k * 16, j * P * 16);
-            w[u * R + 2 * j] = make_float2(v.x, v.y);
-            w[u * R + 2 * j + 1] = make_float2(v.z, v.w);
+            w[u * F + 2 * j] = make_float2(v.x, v.y);
+            w[u * F + 2 * j + 1] = make_float2(v.z, v.w);
           }
         } else {
 #pragma unroll
-          for (int q = 1; q < R; ++q) w[u * R + q] = bld(rs, k * 8, q * P * 8);
+          for (int q = F > 1 ? 1 : 0; q < F; ++q) w[u * F + q] = bld(rs, k * 8, q * P * 8);
         }
       }
     }
   }
 };
 
-template <int N, int T, int SIGN, class Lay, bool PP, int P, int PING, bool SPLIT>
-struct Stages<N, T, SIGN, Lay, PP, P, PING, SPLIT> {
-  using Tw = StageTw<T, 1, 1, 1>;
+template <int N, int T, int SIGN, class Lay, bool PP, int P, int PING, bool SPLIT, bool FUSED>
+struct Stages<N, T, SIGN, Lay, PP, P, PING, SPLIT, FUSED> {
+  using Tw = StageTw<T, 1, 1, 1, false>;
   template <class W>
   static __device__ __forceinline__ void run(float2*, float2*, float2*, const Lay&, int, const float2*, const W&) {}
 };
 
-template <int N, int T, int SIGN, class Lay, bool PP, int P, int PING, bool SPLIT, int R, int... RS>
-struct Stages<N, T, SIGN, Lay, PP, P, PING, SPLIT, R, RS...> {
+template <int N, int T, int SIGN, class Lay, bool PP, int P, int PING, bool SPLIT, bool FUSED, int R, int... RS>
+struct Stages<N, T, SIGN, Lay, PP, P, PING, SPLIT, FUSED, R, RS...> {
   static constexpr int E = N / T;
   static constexpr int U = E / R;
   static_assert(E % R == 0, "radix must divide elements per lane");
   static_assert(T % 16 == 0, "lane count must be a multiple of 16");
   static_assert(!SPLIT || (!PP && E % 2 == 0 && (N / 2) % 16 == 0), "split exchange: one buffer, even E");
   static constexpr bool LAST = sizeof...(RS) == 0;
-  using Tw = StageTw<T, P, R, U>;
-  using Next = Stages<N, T, SIGN, Lay, PP, P * R, PP ? 1 - PING : 0, SPLIT, RS...>;
+  using Tw = StageTw<T, P, R, U, FUSED>;
+  using Next = Stages<N, T, SIGN, Lay, PP, P * R, PP ? 1 - PING : 0, SPLIT, FUSED, RS...>;
 
   // `tw` points at this stage's table; `cur` holds this stage's twiddles.
   static __device__ __forceinline__ void run(float2* x, float2* lds0, float2* lds1, const Lay& lay, int t,
                                              const float2* __restrict__ tw, const Tw& cur) {
     float2* buf = PING ? lds1 : lds0;
-    const float2* tw_next = tw + (P > 1 ? P * R : 0);
+    const float2* tw_next = tw + (P > 1 ? stage_table_len(P * Tw::F) : 0);
     typename Next::Tw nxt;
     if constexpr (!LAST && !TOTEM_TW_LATE) nxt.load(tw_next, t);
     float2 out[E];
@@ -317,15 +391,19 @@ struct Stages<N, T, SIGN, Lay, PP, P, PING, SPLIT, R, RS...> {
       float2 a[R];
 #pragma unroll
       for (int q = 0; q < R; ++q) a[q] = x[u + q * U];
-      if constexpr (P > 1) {
+      if constexpr (P > 1 && fused_stage<R, FUSED>()) {
+        twiddled_dft<R, SIGN>(a, cur.w + u * Tw::F);
+      } else {
+        if constexpr (P > 1) {
 #pragma unroll
-        for (int q = 1; q < R; ++q) {
-          float2 w = cur.w[u * R + q];
-          if (SIGN > 0) w.y = -w.y;
-          a[q] = cmul(a[q], w);
+          for (int q = 1; q < R; ++q) {
+            float2 w = cur.w[u * R + q];
+            if (SIGN > 0) w.y = -w.y;
+            a[q] = cmul(a[q], w);
+          }
         }
+        dft<R, SIGN>(a);
       }
-      dft<R, SIGN>(a);
       if constexpr (LAST || SPLIT) {
         jw[u] = (b - k) * R + k;
 #pragma unroll
@@ -390,10 +468,11 @@ struct Stages<N, T, SIGN, Lay, PP, P, PING, SPLIT, R, RS...> {
 template <int N_, int T_, int... RS> struct PlanDef {
   static constexpr int N = N_;
   static constexpr int T = T_;
+  static constexpr bool FUSED = false;
   static constexpr int NRAD = sizeof...(RS);
   static constexpr int EXCH = NRAD - 1;  // LDS exchanges per transform
-  template <int S, class L, bool PP, int START, bool SPLIT = false>
-  using St = Stages<N, T, S, L, PP, 1, START, SPLIT, RS...>;
+  template <int S, class L, bool PP, int START, bool SPLIT = false, bool FUSED = false>
+  using St = Stages<N, T, S, L, PP, 1, START, SPLIT, FUSED, RS...>;
   static constexpr int radix(int i) {
     constexpr int r[] = {RS...};
     return r[i];
@@ -416,12 +495,18 @@ template <> struct PlanB<1024> : PlanDef<1024, 128, 8, 8, 8, 2> {};  // 8 elemen
 template <> struct PlanB<512> : PlanDef<512, 64, 8, 8, 8> {};          // 8 elements per lane
 template <> struct PlanB<1536> : PlanDef<1536, 128, 4, 4, 4, 4, 2, 3> {};  // 12 elements per lane
 
+// A plan with its even-radix stages after the first in fused form.
+template <class PL> struct Fused : PL {
+  static constexpr bool FUSED = true;
+};
+
 // Number of twiddle entries of a plan's table.
 template <class PL> __host__ __device__ constexpr int plan_twiddle_len() {
   int p = 1, len = 0;
   for (int i = 0; i < PL::NRAD; ++i) {
-    if (p > 1) len += p * PL::radix(i);
-    p *= PL::radix(i);
+    const int r = PL::radix(i);
+    if (p > 1) len += stage_table_len(p * (PL::FUSED && fused_radix(r) ? r / 2 : r));
+    p *= r;
   }
   return len;
 }
@@ -434,7 +519,7 @@ template <int N, int SIGN, bool PP, int START = 0, bool SPLIT = false, class PL 
 __device__ __forceinline__ void block_fft(float2* x, float2* lds0, float2* lds1, const Lay& lay, int t,
                                           const float2* tw) {
   static_assert(PL::N == N, "plan length");
-  using St = typename PL::template St<SIGN, Lay, PP, START, SPLIT>;
+  using St = typename PL::template St<SIGN, Lay, PP, START, SPLIT, PL::FUSED>;
   typename St::Tw none;  // the first stage has no twiddles
   St::run(x, lds0, lds1, lay, t, tw, none);
 }

@@ -94,9 +94,20 @@ namespace totem {
 // the column exchanges run through half buffers.  Variant 0 is the default; the
 // others are chosen at run time per device (totem_stem_set_plan, or measured by
 // totem_stem_autotune), for a whole run or served grid side at a time.
+// Base schedules whose passes run in fused form: the grid sides at which it is no less
+// exact than separate twiddle products, by the exit waves of 80 slices against
+// complex128 (relative L2, separate -> fused; the images' error falls more, by up to a
+// factor of ten, with the balanced factors): 128 2.7e-6 -> 2.5e-6, 512 2.8e-6 -> 2.7e-6,
+// 1024 3.3e-6 -> 3.1e-6, 1536 3.8e-6 -> 3.6e-6.  At 2048 (120 slices) the rows alone
+// 4.2e-6 -> 4.2e-6, both passes 4.5e-6, and the columns pass gains nothing; 256 1.5e-6 ->
+// 2.6e-6 and 768 4.1e-6 -> 4.4e-6 stay separate.  Rows / columns pass, us per launch of
+// the full batch: 512 50.6 / 53.4 -> 48.3 / 51.8, 1024 70.6 / 54.9 -> 63.4 / 51.9 (24
+// probes on average), 2048 rows 88 -> 81.
+constexpr bool fused_cols(int n) { return n == 128 || n == 512 || n == 1024 || n == 1536; }
+constexpr bool fused_rows(int n) { return fused_cols(n) || n == 2048; }
 template <int N> struct PassSpecBase {
-  using RowPlan = Plan<N>;
-  using ColPlan = Plan<N>;
+  using RowPlan = std::conditional_t<fused_rows(N), Fused<Plan<N>>, Plan<N>>;
+  using ColPlan = std::conditional_t<fused_cols(N), Fused<Plan<N>>, Plan<N>>;
   static constexpr int rows_threads = (N == 1024 || N == 768) ? TOTEM_ROWS_THREADS_SMALL
                                       : (N == 2048 && TOTEM_ROWS_SPLIT2048) ? 2 * TOTEM_ROWS_THREADS
                                                                              : TOTEM_ROWS_THREADS;
@@ -1053,7 +1064,9 @@ template <class... PLS> struct PlanSet {
   }
 };
 using AllPlans = PlanSet<Plan<64>, Plan<128>, Plan<256>, Plan<320>, Plan<512>, Plan<768>, Plan<1024>, Plan<1536>,
-                         Plan<2048>, PlanB<768>, PlanB<1024>, PlanB<512>, PlanB<1536>>;
+                         Plan<2048>, Fused<Plan<64>>, Fused<Plan<128>>, Fused<Plan<256>>, Fused<Plan<320>>,
+                         Fused<Plan<512>>, Fused<Plan<768>>, Fused<Plan<1024>>, Fused<Plan<1536>>, Fused<Plan<2048>>,
+                         PlanB<768>, PlanB<1024>, PlanB<512>, PlanB<1536>>;
 __device__ __align__(16) float2 g_twiddles[AllPlans::total];
 
 // Stage (P, R) of a plan, P > 1: the factor exp(-2 pi i q k / (P R)) of input q of a
@@ -1066,9 +1079,22 @@ template <class PL> void twiddle_host_plan(std::vector<float2>& out) {
   int p = 1;
   for (int i = 0; i < PL::NRAD; ++i) {
     const int r = PL::radix(i);
-    if (p > 1) {
+    if (p > 1 && PL::FUSED && fused_radix(r)) {
+      const int f = r / 2;
       const size_t base = out.size();
-      out.resize(base + (size_t)p * r);
+      out.resize(base + (size_t)stage_table_len(p * f), make_float2(0.f, 0.f));
+      std::vector<double> sum(f, 0.0);
+      for (int k = 0; k < p; ++k)
+        for (int q = 0; q < f; ++q) {
+          // w^a W_r^b with w = exp(-2 pi i k / (p r)): angle a k / (p r) + b / r turns
+          const double a = -2.0 * M_PI * ((double)fused_power(r, q, false) * k / (double)(p * r) +
+                                          (double)fused_power(r, q, true) / (double)r);
+          const size_t at = f % 2 == 0 ? ((size_t)(q / 2) * p + k) * 2 + q % 2 : (size_t)q * p + k;
+          out[base + at] = balanced_float2(std::cos(a), std::sin(a), sum[q]);
+        }
+    } else if (p > 1) {
+      const size_t base = out.size();
+      out.resize(base + (size_t)stage_table_len(p * r), make_float2(0.f, 0.f));
       for (int k = 0; k < p; ++k)
         for (int q = 0; q < r; ++q) {
           const double a = -2.0 * M_PI * (double)q * (double)k / (double)(p * r);
