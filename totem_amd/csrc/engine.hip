@@ -1387,16 +1387,16 @@ static void project_impl(const ProjectArgs& a, int paraflag, bool potential_only
     validate_job(probe_check);
   }
   build_transmission_impl(pd, t.as<float2>(), nullptr, nullptr, st);
-  // probes and propagator: double -> complex64 (initKernel_W, cuda_source_lobato.cu:39-57; :1207-1220)
-  std::vector<float2> hp(n2 * M), hh(n2);
-  for (size_t i = 0; i < n2 * M; ++i) hp[i] = make_float2((float)a.my_real_w[i], (float)a.my_imag_w[i]);
-  for (size_t i = 0; i < n2; ++i) {
-    const double re = a.my_real_const[i], im = a.my_img_const[i];
-    hh[i] = std::fabs(re * re + im * im - 1.0) < 1e-12 ? unit_float2(re, im) : make_float2((float)re, (float)im);
-  }
-  DevBuf dprobe, dprop, daper, daper2, ddet;
-  upload(dprobe, hp, st);
-  upload(dprop, hh, st);
+  // probes and propagator: double -> complex64 on the device (initKernel_W, cuda_source_lobato.cu:39-57; :1207-1220)
+  DevBuf dprobe(n2 * M * sizeof(float2)), dprop(n2 * sizeof(float2)), dre(n2 * M * sizeof(double)),
+      dim(n2 * M * sizeof(double)), daper, daper2, ddet;
+  auto to_device = [&](const double* re, const double* im, DevBuf& out, size_t count, bool unit) {
+    HIP_OK(hipMemcpyAsync(dre.p, re, count * sizeof(double), hipMemcpyHostToDevice, st));
+    HIP_OK(hipMemcpyAsync(dim.p, im, count * sizeof(double), hipMemcpyHostToDevice, st));
+    complex64(st, dre.as<double>(), dim.as<double>(), out.as<float2>(), (long)count, unit);
+  };
+  to_device(a.my_real_w, a.my_imag_w, dprobe, n2 * M, false);
+  to_device(a.my_real_const, a.my_img_const, dprop, n2, true);
   daper.alloc(n2 * A * sizeof(double));
   HIP_OK(hipMemcpyAsync(daper.p, a.aper, n2 * A * sizeof(double), hipMemcpyHostToDevice, st));
   if (L > 0) {

@@ -54,6 +54,8 @@ void reduce_det(hipStream_t st, const ItemDev* items, const int* list, int n, co
 // In-place batched 2-D FFT of `batch` n x n complex64 matrices; the column pass
 // writes to dst (may equal data).  epi: 0 plain, 1 transmission exp(i sigma V), 2 scale 1/n^2.
 void fft2d(int n, hipStream_t st, float2* data, float2* dst, int batch, int sign, int epi, float sigma);
+// out[0..n) = complex64 of (re, im); unit: unit-modulus values as unit_float2 rounds them.
+void complex64(hipStream_t st, const double* re, const double* im, float2* out, long n, bool unit);
 // p[0..n) = value (small fill kernels; graph-capture safe, unlike memset nodes)
 void fill(hipStream_t st, float2* p, long n, float re, float im);
 void fill(hipStream_t st, double* p, long n, double v);
