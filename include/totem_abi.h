@@ -145,7 +145,8 @@ typedef struct totem_stem_job {
                             quadrant swap (cuda_source_lobato.cu:1405-1415) */
 } totem_stem_job;
 
-#define TOTEM_RUN_GRAPH 1     /* capture the slice loop of a batch in a hipGraph and replay it */
+#define TOTEM_RUN_GRAPH 1     /* capture the slice loop of a batch in a hipGraph and replay it
+                                 (runs of eight full batches or more; others are launched directly) */
 #define TOTEM_RUN_TIMING 2    /* time every rows/columns pass with HIP events (no graph; synchronises) */
 
 /* Probes in flight per launch that keep their n x n waves inside the GPU's

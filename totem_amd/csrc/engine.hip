@@ -1005,6 +1005,13 @@ struct KernelTimes {
 };
 static thread_local KernelTimes g_times;
 
+// Full batches from which a run with TOTEM_RUN_GRAPH replays a captured slice loop.
+// Below, the loop is launched directly: capturing costs more than the launches, which a
+// full batch's kernels hide (26 probes of 1024^2, 80 slices: 2 batches and a rest 28.2 ms
+// captured twice, 27.4 ms launched; 40 slices of 512^2 8.1 and 7.8 ms; 10 batches of 20
+// slices 27.2 ms either way, and the host thread free).
+constexpr long kGraphReplays = 8;
+
 static void run_stem_impl(const totem_stem_job& j, int batch, int flags, void* ws, size_t ws_bytes, hipStream_t st) {
   validate_job(j);
   const int n = j.n, S = j.slices, A = j.n_aper, L = j.n_mid, M = j.n_probes, D = j.depth;
@@ -1085,8 +1092,10 @@ static void run_stem_impl(const totem_stem_job& j, int batch, int flags, void* w
     ev.resize(2 * S + 1);
     for (auto& e : ev) HIP_OK(hipEventCreate(&e));
   }
+  // A slice loop is captured for the full batches only, and only when enough of them
+  // replay it (kGraphReplays): a capture holds the GPU idle for about 5 us a launch.
+  const bool graph = (flags & TOTEM_RUN_GRAPH) && !(flags & TOTEM_RUN_TIMING) && total / batch >= kGraphReplays;
   hipGraphExec_t gexec = nullptr;
-  int graph_count = -1;
   for (long i0 = 0; i0 < total; i0 += batch) {
     const int cnt = (int)std::min<long>(batch, total - i0);
     const ItemDev* ci = w.items + i0;
@@ -1109,17 +1118,15 @@ static void run_stem_impl(const totem_stem_job& j, int batch, int flags, void* w
         g_times.rows_n += 1;
         g_times.cols_n += 1;
       }
-    } else if (flags & TOTEM_RUN_GRAPH) {
+    } else if (graph && cnt == batch) {
       HIP_OK(hipMemcpyAsync(stage, ci, cnt * sizeof(ItemDev), hipMemcpyDeviceToDevice, st));
-      if (graph_count != cnt) {
-        if (gexec) HIP_OK(hipGraphExecDestroy(gexec));
+      if (!gexec) {
         hipGraph_t g;
         HIP_OK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         record(stage, cnt);
         HIP_OK(hipStreamEndCapture(st, &g));
         HIP_OK(hipGraphInstantiate(&gexec, g, nullptr, nullptr, 0));
         HIP_OK(hipGraphDestroy(g));
-        graph_count = cnt;
       }
       HIP_OK(hipGraphLaunch(gexec, st));
     } else {
@@ -1128,10 +1135,11 @@ static void run_stem_impl(const totem_stem_job& j, int batch, int flags, void* w
     HIP_OK(hipGetLastError());
   }
   for (auto& e : ev) HIP_OK(hipEventDestroy(e));
-  if (gexec) {
-    HIP_OK(hipStreamSynchronize(st));
-    HIP_OK(hipGraphExecDestroy(gexec));
-  }
+  // Runs with TOTEM_RUN_GRAPH end with the stream idle, captured or not: its waves fill the
+  // memory-side cache, and a run that starts on another stream beside them costs both more
+  // than the wait (three 1024^2 runs on three streams 30.8 ms each, one after the other 28.0).
+  if (flags & TOTEM_RUN_GRAPH) HIP_OK(hipStreamSynchronize(st));
+  if (gexec) HIP_OK(hipGraphExecDestroy(gexec));
   if (own.p) HIP_OK(hipStreamSynchronize(st));
 }
 
