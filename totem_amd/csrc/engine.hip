@@ -380,8 +380,9 @@ struct PotDev {
   const PotClass* classes = nullptr;
   int n_classes = 0;
   bool absorptive = false;  // some class has an absorptive part
+  bool corrected = false;   // correction classes: their runs repeat the atoms' own
   const double *tx = nullptr, *ty = nullptr, *wt = nullptr;
-  const PotSeg* segs = nullptr;
+  PotSeg* segs = nullptr;
   std::vector<long> term_off, seg_off;  // host, [S + 1]
   double sigma = 0.0, parameter = 0.0;
   bool sym = false;  // paired frequencies: a quarter of the tiles (hermitian_pairs)
@@ -389,7 +390,7 @@ struct PotDev {
 
 // Scratch of potential builds: phase tables, form factors, slice entries.
 struct PotScratch {
-  DevBuf ex, ey, ff, slices;
+  DevBuf ex, ey, ff, slices, dup;
   size_t bytes() const { return ex.bytes + ey.bytes + ff.bytes; }
   void release() {
     ex.release();
@@ -438,6 +439,12 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
     if (p.absorptive) ff_im = ff_re + (size_t)p.n_classes * np2;
     form_table(st, p.classes, p.n_classes, p.s2, p.corr, np, ff_re, ff_im);
   }
+  unsigned char* dup = nullptr;
+  if (p.corrected && p.term_off[S] > 0) {
+    reserve(sc.dup, p.term_off[S]);
+    dup = sc.dup.as<unsigned char>();
+    repeated_runs(st, sc.slices.as<PotSlice>(), S, p.segs, p.tx, p.ty, p.wt, dup);
+  }
   tw_table(np);
   const float sig = (float)(p.sigma / 1000.0);
   const bool want_v = v_re && v_im;
@@ -447,7 +454,7 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
     const int s0 = chunks[c], cnt = chunks[c + 1] - s0;
     const long t0 = p.term_off[s0];
     float2* tc = t_dev + (size_t)s0 * np2;
-    phase_tables(st, p.tx + t0, p.ty + t0, p.wt + t0, (int)(p.term_off[s0 + cnt] - t0), p.kx1, p.ky1, np, p.sym,
+    phase_tables(st, p.tx + t0, p.ty + t0, p.wt + t0, dup ? dup + t0 : nullptr, (int)(p.term_off[s0 + cnt] - t0), p.kx1, p.ky1, np, p.sym,
                  sc.ex.as<float2>(), sc.ey.as<float2>());
     accumulate(st, sc.ex.as<float2>(), sc.ey.as<float2>(), sc.slices.as<PotSlice>() + s0, cnt, (int)t0, p.segs,
                p.classes, ff_re, ff_im, p.s2, p.aper, p.corr, p.parameter, np, p.sym, tc);
@@ -545,7 +552,10 @@ static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev
   pd.corr = sc->dcorr.as<double>();
   pd.classes = sc->dcls.as<PotClass>();
   pd.n_classes = (int)P.classes.size();
-  for (const PotClass& k : P.classes) pd.absorptive = pd.absorptive || k.has_abs;
+  for (const PotClass& k : P.classes) {
+    pd.absorptive = pd.absorptive || k.has_abs;
+    pd.corrected = pd.corrected || k.kind == kCorr || k.kind == kCorrIon;
+  }
   pd.tx = sc->dtx.as<double>();
   pd.ty = sc->dty.as<double>();
   pd.wt = sc->dwt.as<double>();
@@ -579,7 +589,7 @@ struct totem_specimen {
       wslot, counts, sort_tmp;
   totem::DevBuf tx, ty, wt, segs, classes, kx, ky, s2, aper, corr;
   totem::PotScratch pot;
-  bool absorptive = false;
+  bool absorptive = false, corrected = false;
   std::vector<int> h_counts;
   std::vector<totem::PotSeg> h_segs;
 };
@@ -671,7 +681,10 @@ static totem_specimen* specimen_create_impl(const totem_specimen_desc& d) {
   sp->sigma = d.pot.sigma;
   sp->parameter = d.pot.parameter;
   sp->has_rms = d.rms != nullptr;
-  for (const PotClass& k : classes) sp->absorptive = sp->absorptive || k.has_abs;
+  for (const PotClass& k : classes) {
+    sp->absorptive = sp->absorptive || k.has_abs;
+    sp->corrected = sp->corrected || k.kind == kCorr || k.kind == kCorrIon;
+  }
   sp->sym = hermitian_pairs(P.kx1.data(), P.ky1.data(), np);
   while ((1L << sp->bits) <= (long)S * Ct) ++sp->bits;
   hipStream_t st = lib_stream();
@@ -783,6 +796,7 @@ static void specimen_transmission_impl(totem_specimen& sp, uint64_t seed, int co
   pd.classes = sp.classes.as<PotClass>();
   pd.n_classes = C;
   pd.absorptive = sp.absorptive;
+  pd.corrected = sp.corrected;
   pd.tx = sp.tx.as<double>();
   pd.ty = sp.ty.as<double>();
   pd.wt = sp.wt.as<double>();

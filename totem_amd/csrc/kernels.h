@@ -74,6 +74,8 @@ struct PotClass {
 struct PotSeg {
   int cls;          // class index
   int begin, end;   // term range relative to the slice's first term
+  int next = -1;    // a later run of the slice with the same terms (their sum serves both), or -1
+  int dup = 0;      // 1: an earlier run's sum serves this one
 };
 
 // One slice of a potential build: its first term and its runs of terms.

@@ -740,14 +740,16 @@ k_fft_cols(const float2* __restrict__ src, float2* __restrict__ dst, int epi, fl
 // product k.x is formed and reduced modulo 1 in FP64 before the (FP64) sincospi, and
 // the term's weight is applied in FP64 before the rounding to FP32.  Only the first
 // nc entries of each row are formed and stored (the accumulation reads no more);
-// entries at or beyond np, in the last tile's overhang, are zero.
+// entries at or beyond np, in the last tile's overhang, are zero.  Terms of runs that
+// k_repeated_runs marked are left out: nothing reads them.
 __global__ void __launch_bounds__(256) k_phase(const double* __restrict__ tx, const double* __restrict__ ty,
-                                               const double* __restrict__ wt, const double* __restrict__ kx1,
-                                               const double* __restrict__ ky1, int np, int nc,
-                                               float2* __restrict__ ex, float2* __restrict__ ey) {
+                                               const double* __restrict__ wt,
+                                               const unsigned char* __restrict__ dup,
+                                               const double* __restrict__ kx1, const double* __restrict__ ky1, int np,
+                                               int nc, float2* __restrict__ ex, float2* __restrict__ ey) {
   const int c = blockIdx.y * blockDim.x + threadIdx.x;
   const int j = blockIdx.x;
-  if (c >= nc) return;
+  if (c >= nc || (dup && dup[j])) return;
   const size_t at = (size_t)j * nc + c;
   if (c >= np) {
     ex[at] = ey[at] = make_float2(0.f, 0.f);
@@ -801,6 +803,73 @@ __device__ __forceinline__ double2 form_factor(const PotClass& k, double s2, con
   }
   const double im = k.has_abs ? peng5(k.ab, s2) : 0.0;
   return make_double2(re, im);
+}
+
+// Runs of a slice whose terms repeat an earlier run's (same x, y and weight, in order): an
+// atom's correction term stands beside its own term, at the same place and weight, in
+// another class, and the structure-factor sum, which is most of a build, is the same for
+// both.  Each such run is linked to the earlier one (`next`) and marked (`dup`), its terms
+// in dup[].  One workgroup per slice; runs are compared by length and a hash of their
+// terms' bits, and a match is checked term by term.  Slices of more than kMaxRuns runs are
+// left as they are.
+constexpr int kMaxRuns = 512;
+__global__ void __launch_bounds__(256) k_repeated_runs(const PotSlice* __restrict__ slices, PotSeg* __restrict__ segs,
+                                                       const double* __restrict__ tx, const double* __restrict__ ty,
+                                                       const double* __restrict__ wt,
+                                                       unsigned char* __restrict__ dup) {
+  __shared__ unsigned long long hash[kMaxRuns];
+  __shared__ int same[kMaxRuns], len[kMaxRuns], differ;
+  const PotSlice ps = slices[blockIdx.x];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int n = ps.n_seg <= kMaxRuns ? ps.n_seg : 0;
+  for (int i = 0; i < ps.n_seg; ++i) {
+    const PotSeg sg = segs[ps.seg + i];
+    for (int j = sg.begin + (int)threadIdx.x; j < sg.end; j += 256) dup[ps.term + j] = 0;
+  }
+  for (int i = wave; i < n; i += 4) {
+    const PotSeg sg = segs[ps.seg + i];
+    unsigned long long h = 0;
+    for (int j = sg.begin + lane; j < sg.end; j += 64) {
+      const size_t at = ps.term + j;
+      const unsigned long long v = (unsigned long long)__double_as_longlong(tx[at]) * 0x9E3779B97F4A7C15ull ^
+                                   (unsigned long long)__double_as_longlong(ty[at]) * 0xC2B2AE3D27D4EB4Full ^
+                                   (unsigned long long)__double_as_longlong(wt[at]);
+      h += (v ^ (v >> 29)) * (2ull * (unsigned)(j - sg.begin) + 1ull);
+    }
+    for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);
+    if (lane == 0) {
+      hash[i] = h;
+      len[i] = sg.end - sg.begin;
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += 256) {
+    int f = i;  // first run like run i
+    for (int j = 0; j < i && f == i; ++j)
+      if (hash[j] == hash[i] && len[j] == len[i]) f = j;
+    same[i] = f;
+  }
+  __syncthreads();
+  for (int i = 0; i < n; ++i) {  // uniform over the workgroup
+    const int f = same[i];
+    if (f == i) continue;
+    if (threadIdx.x == 0) differ = 0;
+    __syncthreads();
+    const size_t a = ps.term + segs[ps.seg + f].begin, b = ps.term + segs[ps.seg + i].begin;
+    for (int j = threadIdx.x; j < len[i]; j += 256)
+      if (tx[a + j] != tx[b + j] || ty[a + j] != ty[b + j] || wt[a + j] != wt[b + j]) differ = 1;
+    __syncthreads();
+    if (!differ) {
+      for (int j = threadIdx.x; j < len[i]; j += 256) dup[b + j] = 1;
+      if (threadIdx.x == 0) {  // to the end of run f's chain
+        int k = ps.seg + f;
+        while (segs[k].next >= 0) k = segs[k].next;
+        segs[k].next = ps.seg + i;
+        segs[ps.seg + i].dup = 1;
+      }
+    }
+    __syncthreads();
+  }
 }
 
 // ff_re[cls][pix] (and ff_im where some class is absorptive): the form factors of
@@ -906,6 +975,7 @@ k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey
   }
   for (int sgi = ps.seg; sgi < ps.seg + ps.n_seg; ++sgi) {
     const PotSeg sg = segs[sgi];
+    if (sg.dup) continue;
     const int base = ps.term - term_base;
     floatx16 p1 = {}, p2 = {}, p3 = {}, p4 = {};
     float2 a[U], b[U], an[U], bn[U];
@@ -955,38 +1025,45 @@ k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey
     reduce(0, p1);
     reduce(1, p2);
     double fr[NO], fi[NO];
-    if constexpr (FORM != kFormEval) {
+    auto factors = [&](int cls) {
 #pragma unroll
       for (int o = 0; o < NO; ++o) {
-        const size_t at = sg.cls * np2 + max(pix[o], 0);
+        const size_t at = cls * np2 + max(pix[o], 0);
         fr[o] = ff_re[at];
         if constexpr (FORM == kFormComplex) fi[o] = ff_im[at];
       }
-    }
+    };
+    if constexpr (FORM != kFormEval) factors(sg.cls);
     reduce(2, p3);
     reduce(3, p4);
+    for (int run = sgi, cls = sg.cls;;) {  // the run's class and those of its repetitions
 #pragma unroll
-    for (int u = 0; u < NP; ++u)
+      for (int u = 0; u < NP; ++u)
 #pragma unroll
-      for (int quad = 0; quad < 4; ++quad) {
-        const bool cj_c = quad & 1, cj_r = quad >> 1;
-        const int o = 4 * u + quad;
-        if constexpr (FORM == kFormEval) {
-          if (pix[o] < 0) continue;
-          const double2 f = form_factor(classes[sg.cls], s2v[o], corr, pix[o], np2);
-          fr[o] = f.x;
-          fi[o] = f.y;
+        for (int quad = 0; quad < 4; ++quad) {
+          const bool cj_c = quad & 1, cj_r = quad >> 1;
+          const int o = 4 * u + quad;
+          if constexpr (FORM == kFormEval) {
+            if (pix[o] < 0) continue;
+            const double2 f = form_factor(classes[cls], s2v[o], corr, pix[o], np2);
+            fr[o] = f.x;
+            fi[o] = f.y;
+          }
+          const double sre = cj_r == cj_c ? (double)(q[0][u] - q[1][u]) : (double)(q[0][u] + q[1][u]);
+          const double sim = (double)(cj_c ? -q[2][u] : q[2][u]) + (double)(cj_r ? -q[3][u] : q[3][u]);
+          if constexpr (FORM == kFormRe) {
+            vr[o] += fr[o] * sre;
+            vi[o] += fr[o] * sim;
+          } else {
+            vr[o] += fr[o] * sre - fi[o] * sim;
+            vi[o] += fr[o] * sim + fi[o] * sre;
+          }
         }
-        const double sre = cj_r == cj_c ? (double)(q[0][u] - q[1][u]) : (double)(q[0][u] + q[1][u]);
-        const double sim = (double)(cj_c ? -q[2][u] : q[2][u]) + (double)(cj_r ? -q[3][u] : q[3][u]);
-        if constexpr (FORM == kFormRe) {
-          vr[o] += fr[o] * sre;
-          vi[o] += fr[o] * sim;
-        } else {
-          vr[o] += fr[o] * sre - fi[o] * sim;
-          vi[o] += fr[o] * sim + fi[o] * sre;
-        }
-      }
+      run = segs[run].next;
+      if (run < 0) break;
+      cls = segs[run].cls;
+      if constexpr (FORM != kFormEval) factors(cls);
+    }
   }
   float2* const out = vshift + sl * np2;
 #pragma unroll
@@ -1349,12 +1426,18 @@ bool hermitian_pairs(const double* kx1, const double* ky1, int np) {
 // whole 32-entry tiles of [0, np/2] (paired frequencies) or of [0, np)
 int phase_columns(int np, bool sym) { return ((sym ? np / 2 + 1 : np) + 31) / 32 * 32; }
 
-void phase_tables(hipStream_t st, const double* tx, const double* ty, const double* wt, int n_terms,
-                  const double* kx1, const double* ky1, int np, bool sym, float2* ex, float2* ey) {
+void repeated_runs(hipStream_t st, const PotSlice* slices, int n_slices, PotSeg* segs, const double* tx,
+                   const double* ty, const double* wt, unsigned char* dup) {
+  if (n_slices > 0)
+    hipLaunchKernelGGL(k_repeated_runs, dim3(n_slices), dim3(256), 0, st, slices, segs, tx, ty, wt, dup);
+}
+
+void phase_tables(hipStream_t st, const double* tx, const double* ty, const double* wt, const unsigned char* dup,
+                  int n_terms, const double* kx1, const double* ky1, int np, bool sym, float2* ex, float2* ey) {
   if (n_terms <= 0) return;
   const int nc = phase_columns(np, sym);
-  hipLaunchKernelGGL(k_phase, dim3(n_terms, (nc + 255) / 256), dim3(256), 0, st, tx, ty, wt, kx1, ky1, np, nc, ex,
-                     ey);
+  hipLaunchKernelGGL(k_phase, dim3(n_terms, (nc + 255) / 256), dim3(256), 0, st, tx, ty, wt, dup, kx1, ky1, np, nc,
+                     ex, ey);
 }
 
 void form_table(hipStream_t st, const PotClass* classes, int n_classes, const double* s2, const double* corr, int np,

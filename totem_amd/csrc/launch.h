@@ -65,9 +65,13 @@ void fill(hipStream_t st, double* p, long n, double v);
 bool hermitian_pairs(const double* kx1, const double* ky1, int np);
 // Entries per term of a phase table (whole tiles; about np/2 with paired frequencies).
 int phase_columns(int np, bool sym);
-// ex, ey [n_terms][phase_columns(np, sym)] of the terms.
-void phase_tables(hipStream_t st, const double* tx, const double* ty, const double* wt, int n_terms,
-                  const double* kx1, const double* ky1, int np, bool sym, float2* ex, float2* ey);
+// Links the runs of each slice whose terms repeat an earlier run's (PotSeg::next, dup) and
+// marks their terms in dup (one byte per term of the build).
+void repeated_runs(hipStream_t st, const PotSlice* slices, int n_slices, PotSeg* segs, const double* tx,
+                   const double* ty, const double* wt, unsigned char* dup);
+// ex, ey [n_terms][phase_columns(np, sym)] of the terms (not of those marked in dup, which may be null).
+void phase_tables(hipStream_t st, const double* tx, const double* ty, const double* wt, const unsigned char* dup,
+                  int n_terms, const double* kx1, const double* ky1, int np, bool sym, float2* ex, float2* ey);
 // Form factors of every class at every pixel, ff_re / ff_im [n_classes][np][np] (ff_im may be null).
 void form_table(hipStream_t st, const PotClass* classes, int n_classes, const double* s2, const double* corr, int np,
                 double* ff_re, double* ff_im);
