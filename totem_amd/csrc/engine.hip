@@ -399,10 +399,12 @@ struct PotScratch {
   }
 };
 
-// Phase tables of a chunk of slices (ex and ey together) up to this size, so that the
-// accumulation reads them from the memory-side cache; a slice above it is a chunk of
-// its own.
-constexpr size_t kPhaseChunkBytes = 96ull << 20;
+// Phase tables of a chunk of slices (ex and ey together) up to this size; a slice above
+// it is a chunk of its own. A chunk's last workgroups leave part of the chip idle, so
+// fewer, larger chunks are faster, also beyond the memory-side cache: 80 x 1024^2 slices
+// with corrections 5.6 ms (48 MiB), 4.02 (96), 3.83 (192), 3.66 (384), 3.69 (1024); 30
+// erf-weighted ones of 512^2 2.68, 1.77, 1.66, 1.65, 1.51.
+constexpr size_t kPhaseChunkBytes = 384ull << 20;
 // Form factors are tabulated up to this size.
 constexpr size_t kFormTableBytes = 512ull << 20;
 
@@ -499,7 +501,7 @@ static void flatten_plan(PotentialPlan& P, std::vector<double>& tx, std::vector<
 
 // Builder scratch (phase tables and form factors) above this size is released after
 // the build instead of kept for the next one.
-constexpr size_t kKeepBuilderScratch = 256ull << 20;
+constexpr size_t kKeepBuilderScratch = 512ull << 20;
 
 static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev, double* v_re, double* v_im,
                                     hipStream_t st) {
