@@ -201,13 +201,14 @@ static PotentialPlan plan_potential(const totem_potential_desc& d, bool allow_sp
   P.kx1.assign(d.kx, d.kx + np);
   P.ky1.resize(np);
   for (int r = 0; r < np; ++r) P.ky1[r] = d.ky[(size_t)r * np];
-  for (int r = 0; r < np; ++r)
-    for (int c = 0; c < np; ++c) {
-      const size_t i = (size_t)r * np + c;
-      require(d.kx[i] == P.kx1[c] && d.ky[i] == P.ky1[r],
-              "kx/ky are not meshgrid-separable (kx must vary along columns, ky along rows)",
-              TOTEM_ERR_UNSUPPORTED);
-    }
+  for (int r = 0; r < np; ++r) {
+    // one verdict per row (a check with its message per pixel took most of a small build)
+    const double *kx = d.kx + (size_t)r * np, *ky = d.ky + (size_t)r * np;
+    int same = 1;
+    for (int c = 0; c < np; ++c) same &= (kx[c] == P.kx1[c]) & (ky[c] == P.ky1[r]);
+    require(same != 0, "kx/ky are not meshgrid-separable (kx must vary along columns, ky along rows)",
+            TOTEM_ERR_UNSUPPORTED);
+  }
   const bool lob = d.paraflag == 'l';
   const int ncol = lob ? 14 : 13, ncol_i = lob ? 26 : 25;
   std::map<ClassKey, int> cmap;
