@@ -293,9 +293,8 @@ template <int N, int V> __device__ __forceinline__ void row_lane(int tid, int& l
 // With the remap (unit_map below), XCD x works through the groups
 // [x*G/8, (x+1)*G/8) of every probe in order: neighbouring column groups (which
 // share 128-byte lines) run back to back on one L2, and each L2 only ever sees 1/8
-// of the propagator / a band of the transmission slice.  Any G with G/8 divisible
-// by the units per workgroup gives a bijection; otherwise the plain probe-major
-// order is used.  Taking one group of every probe of the launch in turn instead
+// of the propagator / a band of the transmission slice.  Any G divisible by 8 gives a
+// bijection; otherwise the plain probe-major order is used.  Taking one group of every probe of the launch in turn instead
 // (so that consecutive workgroups of an XCD share a group's transmission rows or
 // propagator columns) measured slower at every size (2048 points, 6 probes per
 // launch: rows 91.5 -> 105 us, columns 108 -> 158 us; 1024: columns 88 -> 120 us).
@@ -311,25 +310,20 @@ __device__ __forceinline__ double wave_sum(double v) {
 #ifndef TOTEM_COLS_HPREFETCH
 #define TOTEM_COLS_HPREFETCH 1  // load the propagator before the forward transform
 #endif
-#ifndef TOTEM_COLS_K
-#define TOTEM_COLS_K 1
-#endif
 
-// Unit u (< K) of workgroup `bid` -> (probe item, group g of G per probe).
-template <int N, int K>
-__device__ __forceinline__ void unit_map(int bid, int u, int G, int& item, int& g) {
+// Workgroup `bid` -> (probe item, group g of G per probe).
+__device__ __forceinline__ void unit_map(int bid, int G, int& item, int& g) {
 #if TOTEM_XCD_REMAP
-  if ((G & 7) == 0 && ((G >> 3) % K) == 0) {
+  if ((G & 7) == 0) {
     const int xcd = bid & 7, gp = G >> 3;
-    const int q = (bid >> 3) * K + u;
+    const int q = bid >> 3;
     item = q / gp;
     g = xcd * gp + (q - item * gp);
     return;
   }
 #endif
-  const int L = bid * K + u;
-  item = L / G;
-  g = L - item * G;
+  item = bid / G;
+  g = bid - item * G;
 }
 
 // The wave source (the probe, row-major, at slice 0; the item's tiled wave after)
@@ -371,7 +365,7 @@ __device__ __forceinline__ RowUnit row_unit(const ItemDev* __restrict__ items, c
   constexpr int RW = Cfg::RW, G = N / RW;
   RowUnit r;
   int item, rg;
-  unit_map<N, K>(blockIdx.x, u, G, item, rg);
+  unit_map(blockIdx.x, G, item, rg);
   const ItemDev it = items[item];
   const JobDev& jb = jobs[it.job];
   r.slice = step - it.start_step;
@@ -513,39 +507,10 @@ __device__ __forceinline__ void detector_partial(const float2* x, const double* 
   __syncthreads();
 }
 
-struct ColUnit {
-  bool active, last;
-  int slice, mid, cg, out;
-  __amdgpu_buffer_rsrc_t wr;
-  const JobDev* jb;
-  double* pbase;
-};
-
-template <int N, int V, int K>
-__device__ __forceinline__ ColUnit col_unit(const ItemDev* __restrict__ items, const JobDev* __restrict__ jobs,
-                                            int step, int u, int groups) {
-  using Cfg = ColCfg<N, V>;
-  constexpr int G = N / Cfg::C;
-  ColUnit r;
-  int item, gi;
-  // `groups` groups per item from the first group of the job's band on (all G groups
-  // with the default band)
-  unit_map<N, K>(blockIdx.x, u, groups, item, gi);
-  const ItemDev it = items[item];
-  r.jb = &jobs[it.job];
-  r.cg = gi + r.jb->band_g0;
-  if (r.cg >= G) r.cg -= G;
-  r.slice = step - it.start_step;
-  // a launch runs the largest band of its jobs; groups beyond a job's own band are idle
-  r.active = r.slice >= 0 && r.slice < r.jb->S && gi < r.jb->band_ng;
-  r.wr = buf_rsrc(it.wave, (unsigned)N * N * sizeof(float2));
-  r.last = r.slice == r.jb->S - 1;
-  r.mid = (r.active && r.jb->mid_of_slice) ? r.jb->mid_of_slice[r.slice] : -1;
-  r.pbase = it.part;
-  r.out = it.out;
-  return r;
-}
-
+// One column group per workgroup, idle ones leaving at once and nothing carried between
+// units (a loop over units, with a flag around each part, kept a second wave's registers
+// and scalars alive: us per launch at the full batch 51.0 -> 49.6 at 1024 points, 50.5 ->
+// 47.4 at 256, 45.1 -> 44.4 at 768).
 // One kernel for every slice; the detector work is a run-time branch (uniform
 // per workgroup).  A variant compiled without the detector code was measured
 // slower at every size (its register allocation gives fewer waves per SIMD:
@@ -557,7 +522,7 @@ k_pass_cols(const ItemDev* __restrict__ items, const JobDev* __restrict__ jobs, 
   using Cfg = ColCfg<N, V>;
   using PL = typename Cfg::PL;
   using Lay = WaveLay<N, V>;
-  constexpr int T = Cfg::T, C = Cfg::C, E = N / T, G = N / C, K = TOTEM_COLS_K;
+  constexpr int T = Cfg::T, C = Cfg::C, E = N / T, G = N / C;
   constexpr int NW = (Cfg::THREADS + 63) / 64;
   constexpr int LC = Cfg::LC;
   static_assert(Cfg::NBUF * LC * sizeof(float2) + NW * kMaxAper * sizeof(double) <= kLdsLimit,
@@ -565,83 +530,62 @@ k_pass_cols(const ItemDev* __restrict__ items, const JobDev* __restrict__ jobs, 
   __shared__ float2 lds[Cfg::NBUF * LC];
   __shared__ double red[NW * kMaxAper];
   float2* const lds1 = lds + (Cfg::NBUF - 1) * LC;
+  constexpr unsigned kBytes = (unsigned)N * N * sizeof(float2);
+  constexpr int kStep = T * N * (int)sizeof(float2);
+  // `groups` groups per item from the first group of the job's band on (all G groups with
+  // the default band); a launch runs the largest band of its jobs, and groups beyond a
+  // job's own band are idle, as is an item before its first slice or after its last
+  int item, gi;
+  unit_map(blockIdx.x, groups, item, gi);
+  const ItemDev it = items[item];
+  const JobDev& jb = jobs[it.job];
+  const int slice = step - it.start_step;
+  if (slice < 0 || slice >= jb.S || gi >= jb.band_ng) return;  // uniform over the workgroup
+  int cg = gi + jb.band_g0;
+  if (cg >= G) cg -= G;
   const int c = threadIdx.x % C;
   const int t = threadIdx.x / C;
   const ColLay<C> lay{c};
-  constexpr unsigned kBytes = (unsigned)N * N * sizeof(float2);
-  constexpr int kStep = T * N * (int)sizeof(float2);
-  float2 xa[E], xb[E];
-  ColUnit ua = col_unit<N, V, K>(items, jobs, step, 0, groups);
+  const int col = cg * C + c;
   // byte offsets of (row t, column): in the wave (WaveLay) and in row-major arrays (H, exit wave);
   // both advance by T*N elements per v
-  int voffa = Lay::at(t, ua.cg * C + c) * (int)sizeof(float2);
-  int hoffa = (t * N + ua.cg * C + c) * (int)sizeof(float2);
-  if (ua.active) {
+  const auto wr = buf_rsrc(it.wave, kBytes);
+  const int voff = Lay::at(t, col) * (int)sizeof(float2);
+  const int hoff = (t * N + col) * (int)sizeof(float2);
+  float2 x[E], hv[TOTEM_COLS_HPREFETCH ? E : 1];
 #pragma unroll
-    for (int v = 0; v < E; ++v) xa[v] = bld(ua.wr, voffa, v * kStep);
+  for (int v = 0; v < E; ++v) x[v] = bld(wr, voff, v * kStep);
+  const auto hr = buf_rsrc(jb.prop, kBytes);
+  // the propagator in column-group order: a wave's 64 lanes read 512 contiguous bytes
+  const bool grouped = jb.prop_cols == C;
+  const int poff = grouped ? ((cg * N + t) * C + c) * (int)sizeof(float2) : hoff;
+  const int pstep = grouped ? T * C * (int)sizeof(float2) : kStep;
+  if constexpr (TOTEM_COLS_HPREFETCH) {
+#pragma unroll
+    for (int v = 0; v < E; ++v) hv[v] = bld(hr, poff, v * pstep);
   }
+  block_fft<N, -1, Cfg::PP, 0, Cfg::SPLIT, PL>(x, lds, lds1, lay, t, tw);
 #pragma unroll
-  for (int u = 0; u < K; ++u) {
-    ColUnit ub;
-    int voffb = 0, hoffb = 0;
-    if (u + 1 < K) {
-      ub = col_unit<N, V, K>(items, jobs, step, u + 1, groups);
-      voffb = Lay::at(t, ub.cg * C + c) * (int)sizeof(float2);
-      hoffb = (t * N + ub.cg * C + c) * (int)sizeof(float2);
-      if (ub.active) {
+  for (int v = 0; v < E; ++v) x[v] = cmul(x[v], TOTEM_COLS_HPREFETCH ? hv[v] : bld(hr, poff, v * pstep));
+  const int mid = jb.mid_of_slice ? jb.mid_of_slice[slice] : -1;
+  if (mid >= 0) {
+    for (int a0 = 0; a0 < jb.A; a0 += kMaxAper)
+      detector_partial<N, E, T, C>(x, jb.aper2 + (size_t)a0 * N * N, false, min(kMaxAper, jb.A - a0), t, col, red,
+                                   it.part + ((size_t)mid * jb.A + a0) * G, G, cg);
+  }
+  if (slice == jb.S - 1) {  // the exit face needs no inverse transform
+    for (int a0 = 0; a0 < jb.A; a0 += kMaxAper)
+      detector_partial<N, E, T, C>(x, jb.aper + (size_t)a0 * N * N, true, min(kMaxAper, jb.A - a0), t, col, red,
+                                   it.part + ((size_t)jb.L * jb.A + a0) * G, G, cg);
+    if (jb.exit) {
+      const auto er = buf_rsrc(jb.exit + (size_t)it.out * N * N, kBytes);
 #pragma unroll
-        for (int v = 0; v < E; ++v) xb[v] = bld(ub.wr, voffb, v * kStep);
-      }
+      for (int v = 0; v < E; ++v) bst(er, hoff, v * kStep, x[v]);
     }
-    if (ua.active) {  // uniform over the workgroup
-      const JobDev& jb = *ua.jb;
-      const int col = ua.cg * C + c;
-      const auto hr = buf_rsrc(jb.prop, kBytes);
-      // the propagator in column-group order: a wave's 64 lanes read 512 contiguous bytes
-      const bool grouped = jb.prop_cols == C;
-      const int poff = grouped ? ((ua.cg * N + t) * C + c) * (int)sizeof(float2) : hoffa;
-      const int pstep = grouped ? T * C * (int)sizeof(float2) : kStep;
-      float2 hv[TOTEM_COLS_HPREFETCH ? E : 1];
-      if constexpr (TOTEM_COLS_HPREFETCH) {
+  } else {
+    block_fft<N, +1, Cfg::PP, next_start<N, Cfg::PP, PL>(0), Cfg::SPLIT, PL>(x, lds, lds1, lay, t, tw);
 #pragma unroll
-        for (int v = 0; v < E; ++v) hv[v] = bld(hr, poff, v * pstep);
-      }
-      block_fft<N, -1, Cfg::PP, 0, Cfg::SPLIT, PL>(xa, lds, lds1, lay, t, tw);
-#pragma unroll
-      for (int v = 0; v < E; ++v) xa[v] = cmul(xa[v], TOTEM_COLS_HPREFETCH ? hv[v] : bld(hr, poff, v * pstep));
-      bool keep = true;
-      {
-        if (ua.mid >= 0) {
-          for (int a0 = 0; a0 < jb.A; a0 += kMaxAper)
-            detector_partial<N, E, T, C>(xa, jb.aper2 + (size_t)a0 * N * N, false, min(kMaxAper, jb.A - a0), t,
-                                         col, red, ua.pbase + ((size_t)ua.mid * jb.A + a0) * G, G, ua.cg);
-        }
-        if (ua.last) {
-          for (int a0 = 0; a0 < jb.A; a0 += kMaxAper)
-            detector_partial<N, E, T, C>(xa, jb.aper + (size_t)a0 * N * N, true, min(kMaxAper, jb.A - a0), t, col,
-                                         red, ua.pbase + ((size_t)jb.L * jb.A + a0) * G, G, ua.cg);
-          keep = false;  // the exit face needs no inverse transform
-          if (jb.exit) {
-            const auto er = buf_rsrc(jb.exit + (size_t)ua.out * N * N, kBytes);
-#pragma unroll
-            for (int v = 0; v < E; ++v) bst(er, hoffa, v * kStep, xa[v]);
-          }
-        }
-      }
-      if (keep) {
-        block_fft<N, +1, Cfg::PP, next_start<N, Cfg::PP, PL>(0), Cfg::SPLIT, PL>(xa, lds, lds1, lay, t, tw);
-#pragma unroll
-        for (int v = 0; v < E; ++v) bst(ua.wr, voffa, v * kStep, xa[v]);
-      }
-      if (u + 1 < K) __syncthreads();  // LDS reuse by the next unit
-    }
-    if (u + 1 < K) {
-      ua = ub;
-      voffa = voffb;
-      hoffa = hoffb;
-#pragma unroll
-      for (int v = 0; v < E; ++v) xa[v] = xb[v];
-    }
+    for (int v = 0; v < E; ++v) bst(wr, voff, v * kStep, x[v]);
   }
 }
 
@@ -708,7 +652,7 @@ k_fft_cols(const float2* __restrict__ src, float2* __restrict__ dst, int epi, fl
   // neighbouring column groups, which share 128-byte lines, run on one XCD's L2 (dispatched
   // round-robin instead, four XCDs fetched and wrote every line: 5 x 1024^2 44.6 us, so 22.6)
   int mat, cg;
-  unit_map<N, 1>(blockIdx.x, 0, G, mat, cg);
+  unit_map(blockIdx.x, G, mat, cg);
   const int c = threadIdx.x % C;
   const int t = threadIdx.x / C;
   const int col = cg * C + c;
@@ -1274,10 +1218,8 @@ template <int N, int V> void launch_pass_rows(hipStream_t st, const ItemDev* ite
 template <int N, int V> void launch_pass_cols(hipStream_t st, const ItemDev* items, int n_items, const JobDev* jobs,
                                               int step, int groups) {
   using Cfg = ColCfg<N, V>;
-  constexpr int K = TOTEM_COLS_K;
-  static_assert((N / Cfg::C) % K == 0, "column groups per probe must be a multiple of K");
-  if (groups <= 0 || groups > N / Cfg::C || groups % K != 0) throw std::runtime_error("columns pass: bad group count");
-  const dim3 grid((unsigned)(n_items * groups / K));
+  if (groups <= 0 || groups > N / Cfg::C) throw std::runtime_error("columns pass: bad group count");
+  const dim3 grid((unsigned)(n_items * groups));
   hipLaunchKernelGGL((k_pass_cols<N, V>), grid, dim3(Cfg::THREADS), 0, st, items, jobs, step, groups,
                      tw_for<typename Cfg::PL>());
 }
