@@ -47,9 +47,16 @@ __device__ __forceinline__ float4 bld4(__amdgpu_buffer_rsrc_t r, int voff, int s
   const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
   return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
 }
+// Cache policy of a store.  kWriteThrough (device scope, SC1): the line goes on to memory
+// when it is written instead of staying dirty in the XCD's L2, so that the end of the
+// launch, which the next launch of the stream waits for, has nothing to write back.  It
+// pays where a launch is short against that write-back (up to 4 MB for each XCD) and
+// where one store instruction covers whole lines; part lines cost a transfer each.
+constexpr int kWriteBack = 0, kWriteThrough = 16;
+template <int POLICY = kWriteBack>
 __device__ __forceinline__ void bst(__amdgpu_buffer_rsrc_t r, int voff, int soff, float2 a) {
   const u32x2 v = {__float_as_uint(a.x), __float_as_uint(a.y)};
-  __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, soff, 0);
+  __builtin_amdgcn_raw_buffer_store_b64(v, r, voff, soff, POLICY);
 }
 
 __device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }

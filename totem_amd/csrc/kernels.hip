@@ -282,6 +282,26 @@ template <int N, int V = 0> constexpr bool rows_wave_local() {
 template <int N, int V> constexpr int rows_lds_pad() {
   return !rows_lane_tiled<N, V>() ? 0 : TOTEM_ROWS_PAD ? TOTEM_ROWS_PAD : 16 / WaveLay<N, V>::TR;
 }
+// How the passes store the wave (kWriteThrough: fft_block.h).  Rows: through where one
+// store instruction covers at least half of each line it touches (the other half comes
+// from the next wave of the workgroup): the wave holds all TR rows of a tile (lane-tiled)
+// or 64 / T of them.  Columns: through where the workgroup's C columns cover a tile's TC;
+// with half lines the other half comes from another workgroup, later.  Both sides of the
+// line, 20 slices, written back -> through (rows and columns as the rule says; us at 1/8 of
+// the full batch, at the full batch): 64 622 -> 435, 3867 -> 3665; 128 680 -> 556, 5476 ->
+// 5309; 256 683 -> 613, 5624 -> 5481; 320 948 -> 836, 7112 -> 7069; 512 744 -> 583, 5280 ->
+// 5247; 768 819 -> 698, 6492 -> 6564; 1024 703 -> 641, 5490 -> 5461; 1536 (columns) 814 ->
+// 818, 7324 -> 7153; 2048 (two probes) 1418 -> 1393, 6420 -> 6403.  Against the rule, full
+// batches: columns through at 768 6647 -> 7096, 1024 5588 -> 6084, 2048 6522 -> 6778, rows
+// through at 1536 7392 -> 7775.  Loads or stores past the caches (nt) cost 10 to 50%.
+template <int N, int V> constexpr int rows_store_policy() {
+  using L = WaveLay<N, V>;
+  constexpr int rows = rows_lane_tiled<N, V>() ? L::TR : 64 / L::RT < 1 ? 1 : 64 / L::RT < L::TR ? 64 / L::RT : L::TR;
+  return rows * L::TC * (int)sizeof(float2) >= 64 ? kWriteThrough : kWriteBack;
+}
+template <int N, int V> constexpr int cols_store_policy() {
+  return ColCfg<N, V>::C >= WaveLay<N, V>::TC ? kWriteThrough : kWriteBack;
+}
 template <int N, int V> __device__ __forceinline__ void row_lane(int tid, int& lr, int& t) {
   constexpr int T = RowCfg<N, V>::T, TR = rows_lane_tiled<N, V>() ? WaveLay<N, V>::TR : 1;
   const int q = tid / (TR * T), rem = tid - q * (TR * T);
@@ -458,7 +478,7 @@ k_pass_rows(const ItemDev* __restrict__ items, const JobDev* __restrict__ jobs, 
       block_fft<N, -1, Cfg::PP, next_start<N, Cfg::PP, PL>(0), Cfg::SPLIT, PL>(xa, lds, lds1, lay, t, tw);
 #pragma unroll
       for (int v = 0; v < E; ++v)  // the columns pass reads band columns only
-        bst(ua.dst, band_off<N, T>(t - ua.lo, v, ua.len, ua.dst_off), DSTEP * v, xa[v]);
+        bst<rows_store_policy<N, V>()>(ua.dst, band_off<N, T>(t - ua.lo, v, ua.len, ua.dst_off), DSTEP * v, xa[v]);
       if (u + 1 < K) __syncthreads();  // LDS reuse by the next unit
     }
     if (u + 1 < K) {
@@ -585,7 +605,7 @@ k_pass_cols(const ItemDev* __restrict__ items, const JobDev* __restrict__ jobs, 
   } else {
     block_fft<N, +1, Cfg::PP, next_start<N, Cfg::PP, PL>(0), Cfg::SPLIT, PL>(x, lds, lds1, lay, t, tw);
 #pragma unroll
-    for (int v = 0; v < E; ++v) bst(wr, voff, v * kStep, x[v]);
+    for (int v = 0; v < E; ++v) bst<cols_store_policy<N, V>()>(wr, voff, v * kStep, x[v]);
   }
 }
 
