@@ -528,8 +528,8 @@ __device__ __forceinline__ void detector_partial(const float2* x, const double* 
 }
 
 // One column group per workgroup, idle ones leaving at once and nothing carried between
-// units (a loop over units, with a flag around each part, kept a second wave's registers
-// and scalars alive: us per launch at the full batch 51.0 -> 49.6 at 1024 points, 50.5 ->
+// units (as a loop over one unit, with a flag around each part and copies for a next unit:
+// us per launch at the full batch 51.0 -> 49.6 at 1024 points, 50.5 ->
 // 47.4 at 256, 45.1 -> 44.4 at 768).
 // One kernel for every slice; the detector work is a run-time branch (uniform
 // per workgroup).  A variant compiled without the detector code was measured

@@ -88,9 +88,11 @@ class DeviceJob:
 
 def footprint_bytes(cfg, M=None, A=None):
     """Device bytes a request holds while in service: transmission stack, probes, propagator,
-    masks and outputs, plus the potential builder's phase tables for its build (about 16 bytes per
-    term and pixel row of the largest slice, counted with the specimen's rows per slice; the
-    builder releases large tables after a build).  Wave slots come from the server's arena."""
+    masks and outputs, plus an allowance for the potential builder's phase tables (16 bytes per
+    term and pixel row of one slice, counted with the specimen's rows per slice).  The builder's
+    scratch is shared by the builds and bounded: 384 MiB of phase tables (more only for a slice
+    that needs it) and 512 MiB of form factors, given back after a build that used more than
+    512 MiB.  Wave slots come from the server's arena."""
     n2, np2 = cfg.n * cfg.n, cfg.np_side * cfg.np_side
     L = len(cfg.mid_slices)
     M = focal_count(cfg) if M is None else M
