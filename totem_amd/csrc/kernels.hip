@@ -609,7 +609,10 @@ k_pass_cols(const ItemDev* __restrict__ items, const JobDev* __restrict__ jobs, 
   }
 }
 
-// Fixed-order Kahan sum of the detector partials of the listed items.
+// Fixed-order Kahan sum of the detector partials of the listed items.  One thread a sum
+// and few threads: bound by the latency of the partials' loads, so 16 are loaded before
+// they are added in turn (one at a time, behind the band test: 28.4 us on average over
+// finishing launches of 256 to 1024 points, so 9.5).
 __global__ void k_reduce_det(const ItemDev* __restrict__ items, const int* __restrict__ list, int n,
                              const JobDev* __restrict__ jobs, int G, int lmax1, int amax) {
   const int idx = blockIdx.x * blockDim.x + threadIdx.x;
@@ -624,15 +627,28 @@ __global__ void k_reduce_det(const ItemDev* __restrict__ items, const int* __res
   if (layer == jb.L || jb.layer_hit[layer]) {
     const double* p = it.part + ((size_t)layer * jb.A + a) * G;
     double comp = 0.0;
-    for (int g = 0; g < G; ++g) {
-      int d = g - jb.band_g0;  // only the job's band groups are written (the rest is zero)
-      if (d < 0) d += G;
-      if (d >= jb.band_ng) continue;
-      const double y = p[g] - comp;
+    auto add = [&](double v) {
+      const double y = v - comp;
       const double tt = s + y;
       comp = (tt - s) - y;
       s = tt;
-    }
+    };
+    // only the job's band groups are written (the rest is zero): in order of g, those of
+    // the band beyond the last group, then the others; a step's partials are loaded together
+    auto sum = [&](int g, int end) {
+      constexpr int U = 16;
+      for (; g + U <= end; g += U) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = p[g + u];
+#pragma unroll
+        for (int u = 0; u < U; ++u) add(v[u]);
+      }
+      for (; g < end; ++g) add(p[g]);
+    };
+    const int past = jb.band_g0 + jb.band_ng;
+    sum(0, min(max(past - G, 0), jb.band_g0));
+    sum(jb.band_g0, min(past, G));
   }
   jb.det[((size_t)layer * jb.A + a) * jb.n_out + it.out] = s;
 }
