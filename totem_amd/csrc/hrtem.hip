@@ -275,6 +275,18 @@ struct HrtemScratch {
   std::map<int, CopyStream> copy;
 };
 
+// Waits for the call's streams when it ends on an error: the copies already queued write
+// the caller's arrays and read the shared scratch, which the next call takes over.
+struct DrainOnError {
+  hipStream_t st, copy = nullptr;
+  bool done = false;
+  ~DrainOnError() {
+    if (done) return;
+    (void)hipStreamSynchronize(st);
+    if (copy) (void)hipStreamSynchronize(copy);
+  }
+};
+
 void reserve_buf(DevBuf& b, size_t bytes) {
   if (b.bytes < bytes) b.alloc(bytes);
 }
@@ -352,6 +364,7 @@ void hrtem_images_impl(const totem_hrtem_desc& d, double* paras_out, double* ima
   reserve_buf(sc.paras, (size_t)B * kPara * sizeof(double));
   reserve_buf(sc.field, (size_t)B * NN * sizeof(float2));
   reserve_buf(sc.img, (size_t)B * NN * sizeof(double));
+  DrainOnError drain{st};
   HIP_OK(hipMemcpyAsync(sc.wave.p, d.wave, NN * sizeof(double2), hipMemcpyHostToDevice, st));
   HIP_OK(hipMemcpyAsync(sc.u.p, d.u, NN * sizeof(double), hipMemcpyHostToDevice, st));
   HIP_OK(hipMemcpyAsync(sc.v.p, d.v, NN * sizeof(double), hipMemcpyHostToDevice, st));
@@ -380,12 +393,14 @@ void hrtem_images_impl(const totem_hrtem_desc& d, double* paras_out, double* ima
     form(0, B);
     HIP_OK(hipMemcpyAsync(images, sc.img.p, (size_t)B * NN * sizeof(double), hipMemcpyDeviceToHost, st));
     HIP_OK(hipStreamSynchronize(st));
+    drain.done = true;
     return;
   }
   int dev = 0;
   HIP_OK(hipGetDevice(&dev));
   CopyStream& copy = sc.copy[dev];
   copy.reserve(chunks);
+  drain.copy = copy.st;
   for (int c = 0; c < chunks; ++c) {
     form(c * per, std::min(per, B - c * per));
     HIP_OK(hipEventRecord(copy.ready[c], st));
@@ -399,6 +414,7 @@ void hrtem_images_impl(const totem_hrtem_desc& d, double* paras_out, double* ima
   }
   HIP_OK(hipStreamSynchronize(copy.st));
   HIP_OK(hipStreamSynchronize(st));
+  drain.done = true;
 }
 
 }  // namespace totem
