@@ -18,6 +18,7 @@
 #include "host_common.h"
 #include "kernels.h"
 #include "launch.h"
+#include "unit_map.h"
 #include "unit_round.h"
 
 #include <algorithm>
@@ -61,9 +62,6 @@
 #endif
 #ifndef TOTEM_COLS_PP
 #define TOTEM_COLS_PP 0
-#endif
-#ifndef TOTEM_XCD_REMAP
-#define TOTEM_XCD_REMAP 1      // XCD-aware workgroup -> (probe, row/column group) mapping
 #endif
 
 namespace totem {
@@ -309,16 +307,6 @@ template <int N, int V> __device__ __forceinline__ void row_lane(int tid, int& l
   t = rem / TR;
 }
 
-// Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2.
-// With the remap (unit_map below), XCD x works through the groups
-// [x*G/8, (x+1)*G/8) of every probe in order: neighbouring column groups (which
-// share 128-byte lines) run back to back on one L2, and each L2 only ever sees 1/8
-// of the propagator / a band of the transmission slice.  Any G divisible by 8 gives a
-// bijection; otherwise the plain probe-major order is used.  Taking one group of every probe of the launch in turn instead
-// (so that consecutive workgroups of an XCD share a group's transmission rows or
-// propagator columns) measured slower at every size (2048 points, 6 probes per
-// launch: rows 91.5 -> 105 us, columns 108 -> 158 us; 1024: columns 88 -> 120 us).
-
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -330,21 +318,6 @@ __device__ __forceinline__ double wave_sum(double v) {
 #ifndef TOTEM_COLS_HPREFETCH
 #define TOTEM_COLS_HPREFETCH 1  // load the propagator before the forward transform
 #endif
-
-// Workgroup `bid` -> (probe item, group g of G per probe).
-__device__ __forceinline__ void unit_map(int bid, int G, int& item, int& g) {
-#if TOTEM_XCD_REMAP
-  if ((G & 7) == 0) {
-    const int xcd = bid & 7, gp = G >> 3;
-    const int q = bid >> 3;
-    item = q / gp;
-    g = xcd * gp + (q - item * gp);
-    return;
-  }
-#endif
-  item = bid / G;
-  g = bid - item * G;
-}
 
 // The wave source (the probe, row-major, at slice 0; the item's tiled wave after)
 // and destination are buffer resources: lanes hold 32-bit byte offsets and the
@@ -385,7 +358,7 @@ __device__ __forceinline__ RowUnit row_unit(const ItemDev* __restrict__ items, c
   constexpr int RW = Cfg::RW, G = N / RW;
   RowUnit r;
   int item, rg;
-  unit_map(blockIdx.x, G, item, rg);
+  unit_map<K>(blockIdx.x, u, G, item, rg);
   const ItemDev it = items[item];
   const JobDev& jb = jobs[it.job];
   r.slice = step - it.start_step;
@@ -556,7 +529,7 @@ k_pass_cols(const ItemDev* __restrict__ items, const JobDev* __restrict__ jobs, 
   // the default band); a launch runs the largest band of its jobs, and groups beyond a
   // job's own band are idle, as is an item before its first slice or after its last
   int item, gi;
-  unit_map(blockIdx.x, groups, item, gi);
+  unit_map(blockIdx.x, 0, groups, item, gi);
   const ItemDev it = items[item];
   const JobDev& jb = jobs[it.job];
   const int slice = step - it.start_step;
@@ -688,7 +661,7 @@ k_fft_cols(const float2* __restrict__ src, float2* __restrict__ dst, int epi, fl
   // neighbouring column groups, which share 128-byte lines, run on one XCD's L2 (dispatched
   // round-robin instead, four XCDs fetched and wrote every line: 5 x 1024^2 44.6 us, so 22.6)
   int mat, cg;
-  unit_map(blockIdx.x, G, mat, cg);
+  unit_map(blockIdx.x, 0, G, mat, cg);
   const int c = threadIdx.x % C;
   const int t = threadIdx.x / C;
   const int col = cg * C + c;
