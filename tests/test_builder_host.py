@@ -1,0 +1,15 @@
+"""The potential builder's host code at its limits, on stand-ins of the HIP calls (tests/hipstub)."""
+import os
+import subprocess
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def test_slice_entries_hold_large_offsets(tmp_path):
+    """Term offsets of a stack are 64-bit throughout: a slice entry takes one beyond 2^31 as it is."""
+    src, exe = tmp_path / "off.cpp", tmp_path / "off"
+    src.write_text('#include <cstdio>\n#include "kernels.h"\nint main() {\n  const long at = 3000000000L;\n'
+                   '  totem::PotSlice s{at, 1, 2};\n  std::printf("%lld\\n", (long long)s.term);\n}\n')
+    subprocess.run(["g++", "-std=c++17", "-Werror=narrowing", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(ROOT, "totem_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout == "3000000000\n"

@@ -426,7 +426,7 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
   std::vector<int> chunks = {0};  // chunk boundaries
   long most = 1;
   for (int s = 0; s < S; ++s) {
-    slices[s] = {(int)p.term_off[s], (int)p.seg_off[s], (int)(p.seg_off[s + 1] - p.seg_off[s])};
+    slices[s] = {p.term_off[s], (int)p.seg_off[s], (int)(p.seg_off[s + 1] - p.seg_off[s])};
     if (s > chunks.back() && p.term_off[s + 1] - p.term_off[chunks.back()] > per_chunk) chunks.push_back(s);
     most = std::max(most, p.term_off[s + 1] - p.term_off[chunks.back()]);
   }
@@ -459,7 +459,7 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
     float2* tc = t_dev + (size_t)s0 * np2;
     phase_tables(st, p.tx + t0, p.ty + t0, p.wt + t0, dup ? dup + t0 : nullptr, (int)(p.term_off[s0 + cnt] - t0), p.kx1, p.ky1, np, p.sym,
                  sc.ex.as<float2>(), sc.ey.as<float2>());
-    accumulate(st, sc.ex.as<float2>(), sc.ey.as<float2>(), sc.slices.as<PotSlice>() + s0, cnt, (int)t0, p.segs,
+    accumulate(st, sc.ex.as<float2>(), sc.ey.as<float2>(), sc.slices.as<PotSlice>() + s0, cnt, t0, p.segs,
                p.classes, ff_re, ff_im, p.s2, p.aper, p.corr, p.parameter, np, p.sym, tc);
     fft2d(np, st, tc, tc, cnt, +1, want_v ? 0 : 1, want_v ? 0.f : sig);
     for (int s = s0; want_v && s < s0 + cnt; ++s) {

@@ -80,7 +80,7 @@ struct PotSeg {
 
 // One slice of a potential build: its first term and its runs of terms.
 struct PotSlice {
-  int term;         // first term in the build's term arrays
+  long term;        // first term in the build's term arrays (a stack may hold more than 2^31)
   int seg, n_seg;   // its PotSeg entries
 };
 

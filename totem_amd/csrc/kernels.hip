@@ -882,7 +882,7 @@ enum FormMode : int { kFormEval, kFormRe, kFormComplex };
 template <int W, int FORM>
 __global__ void __launch_bounds__(64 * W, TOTEM_ACC_MINWAVES)
 k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey, const PotSlice* __restrict__ slices,
-                    int term_base, const PotSeg* __restrict__ segs, const PotClass* __restrict__ classes,
+                    long term_base, const PotSeg* __restrict__ segs, const PotClass* __restrict__ classes,
                     const double* __restrict__ ff_re, const double* __restrict__ ff_im, const double* __restrict__ s2,
                     const double* __restrict__ aper_true, const double* __restrict__ corr, double parameter, int np,
                     int nc, int sym, float2* __restrict__ vshift) {
@@ -929,7 +929,7 @@ k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey
   for (int sgi = ps.seg; sgi < ps.seg + ps.n_seg; ++sgi) {
     const PotSeg sg = segs[sgi];
     if (sg.dup) continue;
-    const int base = ps.term - term_base;
+    const int base = (int)(ps.term - term_base);  // within the chunk
     floatx16 p1 = {}, p2 = {}, p3 = {}, p4 = {};
     float2 a[U], b[U], an[U], bn[U];
     // phases of the group of terms [j, j + GT) (zero beyond the class's last term)
@@ -1404,7 +1404,7 @@ void form_table(hipStream_t st, const PotClass* classes, int n_classes, const do
 #endif
 
 void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSlice* slices, int n_slices,
-                int term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
+                long term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
                 const double* s2, const double* aper_true, const double* corr, double parameter, int np, bool sym,
                 float2* vshift) {
 #define X(S) static_assert(S % 32 == 0 && S <= 32768, "potential tiles: whole tiles without pairs, 32-bit pixels");

@@ -78,7 +78,7 @@ void form_table(hipStream_t st, const PotClass* classes, int n_classes, const do
 // V(k) of slices[0, n_slices) into vshift [n_slices][np][np]; the phase tables start at
 // term `term_base`.  ff_re null: form factors are evaluated per slice and pixel.
 void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSlice* slices, int n_slices,
-                int term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
+                long term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
                 const double* s2, const double* aper_true, const double* corr, double parameter, int np, bool sym,
                 float2* vshift);
 
