@@ -859,18 +859,25 @@ __global__ void __launch_bounds__(256) k_form_table(const PotClass* __restrict__
 // and rows / columns in [1, N/2 - 1] also write their pair N - r: every pixel is
 // written once.  Without it (a grid whose frequencies are not paired) the tiles cover
 // the grid.
-// W waves share a 32 x 32 tile, each taking every W-th group of 8 terms of a class; the
-// partial products are summed in LDS, one product per round through two alternating
-// buffers, and each thread then weights two tile positions' pixels by the class's FP64
-// form factor at each of them.  A 32 x 32 tile reads 512 bytes of phases per term for
-// 4096 multiply-adds, half the operand traffic of a 16 x 16 one, and the next group's
-// phases are in flight during the 16 products of the current one.  Bound by the matrix
-// cores and, behind them, the phases from L2 (about 5 TB/s): a 1024^2 slice of 2000
-// terms takes 64 us, of which 31 us are its products at the FP32 matrix rate (16 x 16
-// tiles with the form factors evaluated in the kernel: 100 us).  Four waves per tile
-// (216 VGPRs, two tiles per CU, so one's reduction overlaps the other's products)
-// measure as eight at 128 VGPRs do, which spill; groups of 8 terms are 5% faster than
-// groups of 4.
+// Four waves share a 32 x 32 tile, each taking every fourth group of 8 terms of a class;
+// their sums meet in LDS, where each thread adds those of four tile positions (elements
+// [4w, 4w + 4) of the wave w) and weights the positions' pixels by the class's FP64 form
+// factor at each of them.  A run of more than 64 terms is summed in two halves: a wave
+// leaves the first half's sums in its own part of the LDS (no barrier) and adds the
+// second's.  FP32 sums of n terms in chains of L are off by about 2.5e-8 sqrt(L / 2), and
+// the halves keep L at n / 8, that of eight waves a tile: V of one class of 400, 1600,
+// 4000, 16000 terms at 256^2 is 2.0e-7, 3.0e-7, 4.2e-7, 7.3e-7 from 64 bits as whole runs
+// in eight waves were, against 2.4e-7, 3.9e-7, 5.7e-7, 1.0e-6 as whole runs in four.
+// Halves cost 1% of an 80 x 1024^2 build and 4% of an erf-weighted 512^2 one, whose runs
+// are 50 to 450 terms; eight waves cost 7% and 9% (one tile per CU, nothing beside its
+// reduction), halves summed in LDS as the runs are 5% and 11%, one 16 x 16 quadrant per
+// wave with all terms (no LDS, twice the operands) 14% and 11%.
+// A 32 x 32 tile reads 512 bytes of phases per term for 4096 multiply-adds, half the
+// operand traffic of a 16 x 16 one, and the next group's phases are in flight during the
+// 16 products of the current one.  Bound by the matrix cores and, behind them, the phases
+// from L2 (about 5 TB/s).  Two tiles per CU (242 VGPRs with tabulated real factors; with
+// complex or evaluated ones 256 and some spills), so one's reduction overlaps the other's
+// products; groups of 8 terms are 5% faster than groups of 4.
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 #ifndef TOTEM_ACC_STEPS
 #define TOTEM_ACC_STEPS 4
@@ -878,18 +885,20 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 #ifndef TOTEM_ACC_MINWAVES
 #define TOTEM_ACC_MINWAVES 2
 #endif
+constexpr int kAccWaves = 4;   // waves sharing a tile
+constexpr int kOneChain = 64;  // runs of more terms are summed in two halves
 enum FormMode : int { kFormEval, kFormRe, kFormComplex };
-template <int W, int FORM>
-__global__ void __launch_bounds__(64 * W, TOTEM_ACC_MINWAVES)
+template <int FORM>
+__global__ void __launch_bounds__(64 * kAccWaves, TOTEM_ACC_MINWAVES)
 k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey, const PotSlice* __restrict__ slices,
                     long term_base, const PotSeg* __restrict__ segs, const PotClass* __restrict__ classes,
                     const double* __restrict__ ff_re, const double* __restrict__ ff_im, const double* __restrict__ s2,
                     const double* __restrict__ aper_true, const double* __restrict__ corr, double parameter, int np,
                     int nc, int sym, float2* __restrict__ vshift) {
-  constexpr int U = TOTEM_ACC_STEPS, GT = 2 * U;  // matrix steps, terms per group
-  constexpr int NT = 64 * W, NP = 1024 / NT, NO = 4 * NP;  // threads; positions and pixels per thread
-  static_assert(NP * NT == 1024, "one or more positions per thread");
-  __shared__ float red[2][W * 1024];  // [buffer][wave][element][lane]
+  constexpr int W = kAccWaves, U = TOTEM_ACC_STEPS, GT = 2 * U;  // waves; matrix steps, terms per group
+  constexpr int NP = 4, NO = 4 * NP;  // tile positions and pixels per thread
+  static_assert(W == 4, "wave w sums accumulator elements [4w, 4w + 4)");
+  __shared__ float4 red[W][4][4][64];  // [wave][product][elements [4q, 4q + 4)][lane]
   static_assert(sizeof(red) <= kLdsLimit, "accumulation LDS above 64 KiB");
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int dt = nc / 32, tiles = dt * dt;
@@ -904,8 +913,7 @@ k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey
   double s2v[FORM == kFormEval ? NO : 1], vr[NO], vi[NO];
 #pragma unroll
   for (int u = 0; u < NP; ++u) {
-    const int pos = threadIdx.x + NT * u, i = pos >> 6, l = pos & 63;
-    const int r = r0 + 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), c = c0 + (l & 31);
+    const int r = r0 + 8 * wave + 4 * (lane >> 5) + u, c = c0 + (lane & 31);
 #pragma unroll
     for (int quad = 0; quad < 4; ++quad) {  // bit 0: column pair, bit 1: row pair
       const bool cj_c = quad & 1, cj_r = quad >> 1;
@@ -930,8 +938,6 @@ k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey
     const PotSeg sg = segs[sgi];
     if (sg.dup) continue;
     const int base = (int)(ps.term - term_base);  // within the chunk
-    floatx16 p1 = {}, p2 = {}, p3 = {}, p4 = {};
-    float2 a[U], b[U], an[U], bn[U];
     // phases of the group of terms [j, j + GT) (zero beyond the class's last term)
     auto load = [&](int j, float2* x, float2* y) {
       const int left = min(max(sg.end - j, 0), GT);
@@ -944,39 +950,51 @@ k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey
         y[u] = bld(rb, ob[u], 0);
       }
     };
+    // this wave's groups of terms before `end`, from j on; a and b hold group j
+    floatx16 p[4];
+    float2 a[U], b[U], an[U], bn[U];
     int j = sg.begin + GT * wave;
-    if (j < sg.end) load(j, a, b);
-    for (; j < sg.end; j += GT * W) {
-      load(j + GT * W, an, bn);
+    auto products = [&](int end) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        p1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].x, p1, 0, 0, 0);
-        p2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].y, p2, 0, 0, 0);
-        p3 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].y, p3, 0, 0, 0);
-        p4 = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].x, p4, 0, 0, 0);
-      }
+      for (int k = 0; k < 4; ++k) p[k] = floatx16{};
+      for (; j < end; j += GT * W) {
+        load(j + GT * W, an, bn);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        a[u] = an[u];
-        b[u] = bn[u];
-      }
-    }
-    float q[4][NP];
-    auto reduce = [&](int k, const floatx16& p) {
-      float* const mine = red[k & 1] + wave * 1024 + lane;
+        for (int u = 0; u < U; ++u) {
+          p[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].x, p[0], 0, 0, 0);
+          p[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].y, p[1], 0, 0, 0);
+          p[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].y, p[2], 0, 0, 0);
+          p[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].x, p[3], 0, 0, 0);
+        }
 #pragma unroll
-      for (int i = 0; i < 16; ++i) mine[64 * i] = p[i];
-      __syncthreads();
-#pragma unroll
-      for (int u = 0; u < NP; ++u) {
-        float t = 0.f;
-#pragma unroll
-        for (int w = 0; w < W; ++w) t += red[k & 1][w * 1024 + threadIdx.x + NT * u];
-        q[k][u] = t;
+        for (int u = 0; u < U; ++u) {
+          a[u] = an[u];
+          b[u] = bn[u];
+        }
       }
     };
-    reduce(0, p1);
-    reduce(1, p2);
+    auto store = [&](bool add) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float4& m = red[wave][k][i][lane];
+          float4 v = make_float4(p[k][4 * i], p[k][4 * i + 1], p[k][4 * i + 2], p[k][4 * i + 3]);
+          if (add) {
+            const float4 h = m;
+            v = make_float4(h.x + v.x, h.y + v.y, h.z + v.z, h.w + v.w);
+          }
+          m = v;
+        }
+    };
+    const int len = sg.end - sg.begin;
+    const bool halves = len > kOneChain;
+    load(j, a, b);
+    if (halves) {
+      products(sg.begin + (len + 2 * GT * W - 1) / (2 * GT * W) * (GT * W));
+      store(false);
+    }
+    products(sg.end);
     double fr[NO], fi[NO];
     auto factors = [&](int cls) {
 #pragma unroll
@@ -987,8 +1005,23 @@ k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey
       }
     };
     if constexpr (FORM != kFormEval) factors(sg.cls);
-    reduce(2, p3);
-    reduce(3, p4);
+    store(halves);
+    __syncthreads();
+    float q[4][NP];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float4 t = red[0][k][wave][lane];
+#pragma unroll
+      for (int w = 1; w < W; ++w) {
+        const float4 v = red[w][k][wave][lane];
+        t = make_float4(t.x + v.x, t.y + v.y, t.z + v.z, t.w + v.w);
+      }
+      q[k][0] = t.x;
+      q[k][1] = t.y;
+      q[k][2] = t.z;
+      q[k][3] = t.w;
+    }
+    __syncthreads();  // read before the next run's sums are stored
     for (int run = sgi, cls = sg.cls;;) {  // the run's class and those of its repetitions
 #pragma unroll
       for (int u = 0; u < NP; ++u)
@@ -1399,10 +1432,6 @@ void form_table(hipStream_t st, const PotClass* classes, int n_classes, const do
                        corr, np2, ff_re, ff_im);
 }
 
-#ifndef TOTEM_ACC_WAVES
-#define TOTEM_ACC_WAVES 4  // waves sharing one potential tile
-#endif
-
 void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSlice* slices, int n_slices,
                 long term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
                 const double* s2, const double* aper_true, const double* corr, double parameter, int np, bool sym,
@@ -1411,15 +1440,14 @@ void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSli
   TOTEM_FOR_SIZES(X)
 #undef X
   const int nc = phase_columns(np, sym), dt = nc / 32;
-  constexpr int W = TOTEM_ACC_WAVES;
   const dim3 grid((unsigned)(n_slices * dt * dt));
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * W), 0, st, ex, ey, slices, term_base, segs, classes, ff_re, ff_im, s2,
+    hipLaunchKernelGGL(kernel, grid, dim3(64 * kAccWaves), 0, st, ex, ey, slices, term_base, segs, classes, ff_re, ff_im, s2,
                        aper_true, corr, parameter, np, nc, sym ? 1 : 0, vshift);
   };
-  if (ff_im) launch(k_accumulate_mfma32<W, kFormComplex>);
-  else if (ff_re) launch(k_accumulate_mfma32<W, kFormRe>);
-  else launch(k_accumulate_mfma32<W, kFormEval>);
+  if (ff_im) launch(k_accumulate_mfma32<kFormComplex>);
+  else if (ff_re) launch(k_accumulate_mfma32<kFormRe>);
+  else launch(k_accumulate_mfma32<kFormEval>);
 }
 
 }  // namespace totem
