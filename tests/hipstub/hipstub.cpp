@@ -181,6 +181,23 @@ hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) {
 }
 
 // ------------------------------------------------------------------------- kernels, errors
+struct Config {
+  dim3 grid, block;
+  size_t shared;
+  hipStream_t stream;
+};
+static thread_local Config config;
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shared, hipStream_t s) {
+  config = {grid, block, shared, s};
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hipStream_t* s) {
+  *grid = config.grid;
+  *block = config.block;
+  *shared = config.shared;
+  *s = config.stream;
+  return hipSuccess;
+}
 hipError_t hipLaunchKernel(const void*, dim3 grid, dim3 block, void**, size_t, hipStream_t) {
   std::lock_guard<std::mutex> lk(mu);
   ++launches;

@@ -2,6 +2,8 @@
 import os
 import subprocess
 
+from tests import hipstub
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
@@ -13,3 +15,19 @@ def test_slice_entries_hold_large_offsets(tmp_path):
     subprocess.run(["g++", "-std=c++17", "-Werror=narrowing", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                     "-I" + os.path.join(ROOT, "totem_amd", "csrc"), str(src), "-o", str(exe)], check=True)
     assert subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout == "3000000000\n"
+
+
+MANY_SLICES = """
+S, n = 4200000, 64                               # 2^32 threads and more in one launch
+gx, gy, s2 = optics.reciprocal_grids(n, 0.1)
+counts = np.zeros(S)
+counts[[0, 17, S - 1]] = 3
+rows = np.random.default_rng(0).uniform(0.1, 1, (9, 14))
+engine.build_transmission("l", n, S, counts, rows, gx, gy, s2, np.ones_like(s2), 0.7, 1.0, 1 << 40)
+assert stub.stub_widest() < 1 << 32
+"""
+
+
+def test_stack_of_millions_of_small_slices(tmp_path):
+    """A stack of more slices than one launch can hold is built in several."""
+    hipstub.run(tmp_path, MANY_SLICES)

@@ -406,6 +406,9 @@ struct PotScratch {
 // with corrections 5.6 ms (48 MiB), 4.02 (96), 3.83 (192), 3.66 (384), 3.69 (1024); 30
 // erf-weighted ones of 512^2 2.68, 1.77, 1.66, 1.65, 1.51.
 constexpr size_t kPhaseChunkBytes = 384ull << 20;
+// Slices of a chunk, however few terms they hold: a launch's threads are counted in 32
+// bits, and a 2048^2 slice without frequency pairs takes 2^20 of them.
+constexpr int kChunkSlices = 2048;
 // Form factors are tabulated up to this size.
 constexpr size_t kFormTableBytes = 512ull << 20;
 
@@ -427,7 +430,9 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
   long most = 1;
   for (int s = 0; s < S; ++s) {
     slices[s] = {p.term_off[s], (int)p.seg_off[s], (int)(p.seg_off[s + 1] - p.seg_off[s])};
-    if (s > chunks.back() && p.term_off[s + 1] - p.term_off[chunks.back()] > per_chunk) chunks.push_back(s);
+    const int first = chunks.back();
+    if (s > first && (p.term_off[s + 1] - p.term_off[first] > per_chunk || s - first == kChunkSlices))
+      chunks.push_back(s);
     most = std::max(most, p.term_off[s + 1] - p.term_off[chunks.back()]);
   }
   chunks.push_back(S);
