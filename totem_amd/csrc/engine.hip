@@ -389,14 +389,27 @@ struct PotDev {
   bool sym = false;  // paired frequencies: a quarter of the tiles (hermitian_pairs)
 };
 
-// Scratch of potential builds: phase tables, form factors, slice entries.
+// Builder scratch above this size is released after the build instead of kept for the
+// next one, that of builds from rows and of each resident specimen alike.
+constexpr size_t kKeepBuilderScratch = 512ull << 20;
+
+// Scratch of potential builds: phase tables, form factors, slice entries, marks of
+// repeated terms.
 struct PotScratch {
   DevBuf ex, ey, ff, slices, dup;
-  size_t bytes() const { return ex.bytes + ey.bytes + ff.bytes; }
+  size_t bytes() const { return ex.bytes + ey.bytes + ff.bytes + slices.bytes + dup.bytes; }
   void release() {
-    ex.release();
-    ey.release();
-    ff.release();
+    for (DevBuf* b : {&ex, &ey, &ff, &slices, &dup}) b->release();
+  }
+};
+// Ends a build's use of the scratch, also when the build fails: nothing queued on the
+// stream reads it any more, and a large one is given back.
+struct ScratchUse {
+  PotScratch& sc;
+  hipStream_t st;
+  ~ScratchUse() {
+    (void)hipStreamSynchronize(st);
+    if (sc.bytes() > kKeepBuilderScratch) sc.release();
   }
 };
 
@@ -425,6 +438,7 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
   const size_t np2 = (size_t)np * np;
   const size_t term_bytes = 2 * (size_t)phase_columns(np, p.sym) * sizeof(float2);
   const long per_chunk = std::max<long>(1, (long)(kPhaseChunkBytes / term_bytes));
+  ScratchUse use{sc, st};
   std::vector<PotSlice> slices(S);
   std::vector<int> chunks = {0};  // chunk boundaries
   long most = 1;
@@ -505,10 +519,6 @@ static void flatten_plan(PotentialPlan& P, std::vector<double>& tx, std::vector<
   }
 }
 
-// Builder scratch (phase tables and form factors) above this size is released after
-// the build instead of kept for the next one.
-constexpr size_t kKeepBuilderScratch = 512ull << 20;
-
 static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev, double* v_re, double* v_im,
                                     hipStream_t st) {
   PotentialPlan P = plan_potential(d);
@@ -572,7 +582,6 @@ static void build_transmission_impl(const totem_potential_desc& d, float2* t_dev
   pd.parameter = d.parameter;
   pd.sym = hermitian_pairs(P.kx1.data(), P.ky1.data(), P.np);
   potential_run(pd, t_dev, v_re, v_im, st, sc->pot);
-  if (sc->pot.bytes() > kKeepBuilderScratch) sc->pot.release();
 }
 
 // ------------------------------------------------------- specimen on the device
