@@ -59,3 +59,28 @@ assert stub.stub_in_use() - before <= 512 << 20
 def test_specimen_gives_large_scratch_back(tmp_path):
     """A resident specimen keeps no more than 512 MiB of builder scratch between its builds."""
     print(hipstub.run(tmp_path, SPECIMEN))
+
+
+NEARLY_FULL = """
+S, each, n = 40, 2000, 512                       # 9 MB of phase tables a slice, 369 MB the stack
+rng = np.random.default_rng(2)
+gx, gy, s2 = optics.reciprocal_grids(n, 0.1)
+rows = rng.uniform(1, 2, (S * each, 14))
+rows[:, 3:] = rows[0, 3:]
+def build():
+    engine.build_transmission("l", n, S, np.full(S, float(each)), rows, gx, gy, s2, np.ones_like(s2), 0.7, 1.0, 1 << 40)
+need = 2 * each * (n // 2 + 32) * 8              # the tables of one slice
+inputs = 24 * S * each + 3 * 8 * n * n           # terms, s2, AperTrue
+stub.stub_capacity(stub.stub_in_use() + inputs + need + (1 << 20))
+build()
+launches = stub.stub_launches()
+build()
+print("launches", stub.stub_launches() - launches)
+stub.stub_capacity(stub.stub_in_use() + (4 << 30))
+build()
+"""
+
+
+def test_build_on_a_nearly_full_device(tmp_path):
+    """Where the tables of several slices don't fit the device, a stack is built slice by slice."""
+    assert "launches 160" in hipstub.run(tmp_path, NEARLY_FULL)      # four a slice

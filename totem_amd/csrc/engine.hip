@@ -440,23 +440,39 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
   const long per_chunk = std::max<long>(1, (long)(kPhaseChunkBytes / term_bytes));
   ScratchUse use{sc, st};
   std::vector<PotSlice> slices(S);
-  std::vector<int> chunks = {0};  // chunk boundaries
-  long most = 1;
-  for (int s = 0; s < S; ++s) {
+  for (int s = 0; s < S; ++s)
     slices[s] = {p.term_off[s], (int)p.seg_off[s], (int)(p.seg_off[s + 1] - p.seg_off[s])};
-    const int first = chunks.back();
-    if (s > first && (p.term_off[s + 1] - p.term_off[first] > per_chunk || s - first == kChunkSlices))
-      chunks.push_back(s);
-    most = std::max(most, p.term_off[s + 1] - p.term_off[chunks.back()]);
-  }
-  chunks.push_back(S);
-  reserve(sc.ex, most * (term_bytes / 2));
-  reserve(sc.ey, most * (term_bytes / 2));
+  std::vector<int> chunks;  // chunk boundaries
+  auto reserve_tables = [&](long terms, size_t ff_bytes) {  // for chunks of so many terms or one slice
+    chunks = {0};
+    long most = 1;
+    for (int s = 0; s < S; ++s) {
+      const int first = chunks.back();
+      if (s > first && (p.term_off[s + 1] - p.term_off[first] > terms || s - first == kChunkSlices))
+        chunks.push_back(s);
+      most = std::max(most, p.term_off[s + 1] - p.term_off[chunks.back()]);
+    }
+    chunks.push_back(S);
+    reserve(sc.ex, most * (term_bytes / 2));
+    reserve(sc.ey, most * (term_bytes / 2));
+    if (ff_bytes > 0) reserve(sc.ff, ff_bytes);
+  };
   upload(sc.slices, slices, st);
   const size_t ff_bytes = (size_t)p.n_classes * np2 * sizeof(double) * (p.absorptive ? 2 : 1);
+  bool tabulated = p.seg_off[S] >= 2L * p.n_classes && ff_bytes > 0 && ff_bytes <= kFormTableBytes;
+  try {
+    reserve_tables(per_chunk, tabulated ? ff_bytes : 0);
+  } catch (const Error& e) {
+    // a nearly full device: one slice at a time, form factors formed in each, as much
+    // scratch as the largest slice needs
+    if (e.code != TOTEM_ERR_MEMORY) throw;
+    (void)hipGetLastError();
+    for (DevBuf* b : {&sc.ex, &sc.ey, &sc.ff}) b->release();
+    tabulated = false;
+    reserve_tables(1, 0);
+  }
   double *ff_re = nullptr, *ff_im = nullptr;
-  if (p.seg_off[S] >= 2L * p.n_classes && ff_bytes > 0 && ff_bytes <= kFormTableBytes) {
-    reserve(sc.ff, ff_bytes);
+  if (tabulated) {
     ff_re = sc.ff.as<double>();
     if (p.absorptive) ff_im = ff_re + (size_t)p.n_classes * np2;
     form_table(st, p.classes, p.n_classes, p.s2, p.corr, np, ff_re, ff_im);
