@@ -89,10 +89,9 @@ class DeviceJob:
 def footprint_bytes(cfg, M=None, A=None):
     """Device bytes a request holds while in service: transmission stack, probes, propagator,
     masks and outputs, plus an allowance for the potential builder's phase tables (16 bytes per
-    term and pixel row of one slice, counted with the specimen's rows per slice).  The builder's
-    scratch is shared by the builds and bounded: 384 MiB of phase tables (more only for a slice
-    that needs it) and 512 MiB of form factors, given back after a build that used more than
-    512 MiB.  Wave slots come from the server's arena."""
+    term and pixel row of one slice, counted with the specimen's rows per slice).  What the
+    builder's scratch takes beyond that, once for all requests, is :func:`scratch_bytes`.  Wave
+    slots come from the server's arena."""
     n2, np2 = cfg.n * cfg.n, cfg.np_side * cfg.np_side
     L = len(cfg.mid_slices)
     M = focal_count(cfg) if M is None else M
@@ -100,6 +99,39 @@ def footprint_bytes(cfg, M=None, A=None):
     rows = 2 * len(cfg.atoms) / max(cfg.n_slices, 1) + 64     # corrections double the rows
     build = int(16 * rows * cfg.np_side)
     return int(8 * cfg.n_slices * np2 + 8 * M * n2 + 8 * n2 + 16 * A * n2 + 8 * (L + 1) * A * M * cfg.depth) + build
+
+
+def scratch_bytes(cfg):
+    """Bound of the potential builder's scratch for a request's build: phase tables of a chunk of
+    slices (up to 384 MiB, more only for a slice that needs it) and form factors of every class
+    (up to 512 MiB).  One build at a time uses it; a scratch above 512 MiB is given back."""
+    x = np.asarray(cfg.atoms, dtype=np.float64)
+    term = 16 * (-(-(cfg.np_side // 2 + 1) // 32) * 32)
+    rows = 2 * len(x)                                         # corrections double the rows
+    phases = max(min(384 << 20, term * rows), term * (rows // max(cfg.n_slices, 1) + 64))
+    if cfg.multiceng:                                         # rows with coefficients of their own near faces
+        return int(phases) + (512 << 20)
+    classes = 2 * len(np.unique(x[:, [0, 4, 5, 6]], axis=0)) if len(x) else 0
+    return int(phases + min(512 << 20, 8 * classes * cfg.np_side ** 2))
+
+
+class Admission:
+    """Device bytes of the requests in service against a budget: every request's footprint, and the
+    builder's scratch once, at the largest of the requests so far."""
+
+    def __init__(self, budget):
+        self.budget, self.resident, self.peak, self.scratch = budget, 0, 0, 0
+
+    def fits(self, cfg):
+        return self.resident + footprint_bytes(cfg) + max(self.scratch, scratch_bytes(cfg)) <= self.budget
+
+    def take(self, cfg):
+        self.resident += footprint_bytes(cfg)
+        self.peak = max(self.peak, self.resident)
+        self.scratch = max(self.scratch, scratch_bytes(cfg))
+
+    def release(self, cfg):
+        self.resident -= footprint_bytes(cfg)
 
 
 def focal_count(cfg):
@@ -202,8 +234,8 @@ def serve(requests, server, hbm_budget, max_wall=600.0, on_done=None):
     """Run the requests (sorted by ``arrival``, seconds after the start) through ``server``.
 
     A request is admitted when it has arrived and its footprint fits ``hbm_budget`` next to the
-    requests in service or being built (first come, first served; a request larger than the budget
-    is admitted alone).  A builder thread prepares admitted requests (``stem.prepare`` when
+    requests in service or being built and the builder's scratch (first come, first served; a
+    request larger than the budget is admitted alone).  A builder thread prepares admitted requests (``stem.prepare`` when
     ``inp`` is None) and builds their transmission stacks on its own stream; the loop submits each
     one when its build is complete and keeps stepping the server in between.  Returns (wall
     seconds, peak resident bytes); each request gets ``admitted``, ``built``, ``done`` (seconds),
@@ -239,7 +271,7 @@ def serve(requests, server, hbm_budget, max_wall=600.0, on_done=None):
     th = threading.Thread(target=builder, name="totem-serve-builder", daemon=True)
     th.start()
     building = 0
-    resident = peak = 0
+    memory = Admission(hbm_budget)
     try:
         while waiting or arrived or in_service or building:
             now = time.perf_counter() - t0
@@ -249,14 +281,12 @@ def serve(requests, server, hbm_budget, max_wall=600.0, on_done=None):
                 arrived.append(waiting.popleft())
             while arrived:
                 r = arrived[0]
-                fp = footprint_bytes(r.cfg)
-                if (in_service or building) and resident + fp > hbm_budget:
+                if (in_service or building) and not memory.fits(r.cfg):
                     r.extra["budget_wait"] = True
                     break
                 arrived.popleft()
                 r.admitted = time.perf_counter() - t0
-                resident += fp
-                peak = max(peak, resident)
+                memory.take(r.cfg)
                 building += 1
                 todo.put(r)
             while True:
@@ -275,7 +305,7 @@ def serve(requests, server, hbm_budget, max_wall=600.0, on_done=None):
                     r = in_service.pop(jid)
                     r.result = r.job.images()
                     r.done = time.perf_counter() - t0
-                    resident -= footprint_bytes(r.cfg)
+                    memory.release(r.cfg)
                     if on_done:
                         on_done(r)
                     r.job = None
@@ -286,4 +316,4 @@ def serve(requests, server, hbm_budget, max_wall=600.0, on_done=None):
         todo.put(None)
         th.join()
     torch.cuda.synchronize()
-    return time.perf_counter() - t0, peak
+    return time.perf_counter() - t0, memory.peak
