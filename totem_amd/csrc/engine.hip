@@ -1389,6 +1389,10 @@ static void zero_outputs(const ProjectArgs& a, bool potential_only) {
   }
 }
 
+// Values of the FP64 staging of probes and propagator (two of 32 MiB at most, or one
+// probe's): on the device the conversion needs 16 bytes a value beside the 8 kept.
+constexpr size_t kStageValues = 4u << 20;
+
 static void project_impl(const ProjectArgs& a, int paraflag, bool potential_only) {
   zero_outputs(a, potential_only);
   require(a.P_Height == a.P_Width, "P_Height must equal P_Width (square potential grid)");
@@ -1443,15 +1447,24 @@ static void project_impl(const ProjectArgs& a, int paraflag, bool potential_only
   }
   build_transmission_impl(pd, t.as<float2>(), nullptr, nullptr, st);
   // probes and propagator: double -> complex64 on the device (initKernel_W, cuda_source_lobato.cu:39-57; :1207-1220)
-  DevBuf dprobe(n2 * M * sizeof(float2)), dprop(n2 * sizeof(float2)), dre(n2 * M * sizeof(double)),
-      dim(n2 * M * sizeof(double)), daper, daper2, ddet;
-  auto to_device = [&](const double* re, const double* im, DevBuf& out, size_t count, bool unit) {
-    HIP_OK(hipMemcpyAsync(dre.p, re, count * sizeof(double), hipMemcpyHostToDevice, st));
-    HIP_OK(hipMemcpyAsync(dim.p, im, count * sizeof(double), hipMemcpyHostToDevice, st));
-    complex64(st, dre.as<double>(), dim.as<double>(), out.as<float2>(), (long)count, unit);
-  };
-  to_device(a.my_real_w, a.my_imag_w, dprobe, n2 * M, false);
-  to_device(a.my_real_const, a.my_img_const, dprop, n2, true);
+  // through a staging pair of bounded size, given back before the batch is sized by free memory
+  DevBuf dprobe(n2 * M * sizeof(float2)), dprop(n2 * sizeof(float2)), daper, daper2, ddet;
+  {
+    const size_t per = std::min(n2 * M, std::max(n2, kStageValues));
+    DevBuf dre(per * sizeof(double)), dim(per * sizeof(double));
+    auto to_device = [&](const double* re, const double* im, DevBuf& out, size_t count, bool unit) {
+      for (size_t at = 0; at < count; at += per) {
+        const size_t part = std::min(per, count - at);
+        HIP_OK(hipMemcpyAsync(dre.p, re + at, part * sizeof(double), hipMemcpyHostToDevice, st));
+        HIP_OK(hipMemcpyAsync(dim.p, im + at, part * sizeof(double), hipMemcpyHostToDevice, st));
+        complex64(st, dre.as<double>(), dim.as<double>(), out.as<float2>() + at, (long)part, unit);
+      }
+    };
+    to_device(a.my_real_w, a.my_imag_w, dprobe, n2 * M, false);
+    to_device(a.my_real_const, a.my_img_const, dprop, n2, true);
+    HIP_OK(hipGetLastError());
+    HIP_OK(hipStreamSynchronize(st));
+  }
   daper.alloc(n2 * A * sizeof(double));
   HIP_OK(hipMemcpyAsync(daper.p, a.aper, n2 * A * sizeof(double), hipMemcpyHostToDevice, st));
   if (L > 0) {
