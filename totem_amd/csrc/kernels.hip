@@ -97,8 +97,8 @@ namespace totem {
 // complex128 (relative L2, separate -> fused; the images' error falls more, by up to a
 // factor of ten, with the balanced factors): 128 2.7e-6 -> 2.5e-6, 512 2.8e-6 -> 2.7e-6,
 // 1024 3.3e-6 -> 3.1e-6, 1536 3.8e-6 -> 3.6e-6.  At 2048 (120 slices) the rows alone
-// 4.2e-6 -> 4.2e-6, both passes 4.5e-6, and the columns pass gains nothing; 256 1.5e-6 ->
-// 2.6e-6 and 768 4.1e-6 -> 4.4e-6 stay separate.  Rows / columns pass, us per launch of
+// 4.2e-6 -> 4.2e-6, both passes 4.5e-6, and the columns pass gains nothing; 64 2.1e-6 ->
+// 3.0e-6, 256 1.5e-6 -> 2.6e-6, 320 4.1e-6 -> 4.9e-6 and 768 4.1e-6 -> 4.4e-6 stay separate.  Rows / columns pass, us per launch of
 // the full batch: 512 50.6 / 53.4 -> 48.3 / 51.8, 1024 70.6 / 54.9 -> 63.4 / 51.9 (24
 // probes on average), 2048 rows 88 -> 81.
 constexpr bool fused_cols(int n) { return n == 128 || n == 512 || n == 1024 || n == 1536; }
@@ -1163,9 +1163,8 @@ template <class... PLS> struct PlanSet {
   }
 };
 using AllPlans = PlanSet<Plan<64>, Plan<128>, Plan<256>, Plan<320>, Plan<512>, Plan<768>, Plan<1024>, Plan<1536>,
-                         Plan<2048>, Fused<Plan<64>>, Fused<Plan<128>>, Fused<Plan<256>>, Fused<Plan<320>>,
-                         Fused<Plan<512>>, Fused<Plan<768>>, Fused<Plan<1024>>, Fused<Plan<1536>>, Fused<Plan<2048>>,
-                         PlanB<768>, PlanB<1024>, PlanB<512>, PlanB<1536>>;
+                         Plan<2048>, Fused<Plan<128>>, Fused<Plan<512>>, Fused<Plan<1024>>, Fused<Plan<1536>>,
+                         Fused<Plan<2048>>, PlanB<768>, PlanB<1024>, PlanB<512>, PlanB<1536>>;
 __device__ __align__(16) float2 g_twiddles[AllPlans::total];
 
 // Stage (P, R) of a plan, P > 1: the factor exp(-2 pi i q k / (P R)) of input q of a
