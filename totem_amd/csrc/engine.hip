@@ -166,9 +166,14 @@ struct PotentialPlan {
   bool split = false;  // Peng rows split into per-Gaussian classes
 };
 
-// Relative cost of a plan's accumulation: per slice and class present, the
-// class's terms padded to the 16-term groups of the matrix-core sum, plus one
-// FP64 form-factor evaluation per pixel counted as kFormFactorTerms terms.
+// Relative cost of a plan's accumulation: per slice and class present, the class's
+// terms in groups of 16, plus a run's own cost (reduction, form factors per pixel)
+// counted as kFormFactorTerms terms.  A rough model that only has to tell plans of about
+// one class a row from plans of shared classes, which lie far apart.  Builds from rows,
+// rows kept whole / split: erf-weighted rows 256^2 x 10 slices 3.95 / 1.09 ms, 512^2 x 16
+// 39.2 / 8.5, 1024^2 x 8 73 / 6.7, with corrections 512^2 x 8 14.1 / 2.7 (split by the
+// rule); a B of its own per row 256^2 x 10 2.39 / 5.18, 512^2 x 6 3.21 / 6.96 (kept
+// whole); of twelve such builds the rule missed one, a single cell at 256^2 (0.31 / 0.24).
 constexpr long kFormFactorTerms = 32;
 static long plan_cost(const std::vector<std::vector<Term>>& slices, size_t n_classes) {
   std::vector<int> cnt(n_classes, 0);
@@ -1054,9 +1059,10 @@ static thread_local KernelTimes g_times;
 
 // Full batches from which a run with TOTEM_RUN_GRAPH replays a captured slice loop.
 // Below, the loop is launched directly: capturing costs more than the launches, which a
-// full batch's kernels hide (26 probes of 1024^2, 80 slices: 2 batches and a rest 28.2 ms
-// captured twice, 27.4 ms launched; 40 slices of 512^2 8.1 and 7.8 ms; 10 batches of 20
-// slices 27.2 ms either way, and the host thread free).
+// full batch's kernels hide.  A captured run over a launched one, by full batches (20 or 40
+// slices): 256^2 x 64 probes 1.05 (4 batches), 1.03 (6), 1.02 (8), 1.02 (16); 512^2 x 26
+// 1.03, 1.02, 1.01, 1.01; 1024^2 x 26 0.99 to 1.00 throughout.  From eight on capturing
+// costs at most 2%, none at the full batch of 1024^2, and the host thread is free.
 constexpr long kGraphReplays = 8;
 
 static void run_stem_impl(const totem_stem_job& j, int batch, int flags, void* ws, size_t ws_bytes, hipStream_t st) {
@@ -1489,7 +1495,7 @@ static void project_impl(const ProjectArgs& a, int paraflag, bool potential_only
   long batch = (long)(fr / 2 / std::max<size_t>(per, 1));
   batch = std::max<long>(1, std::min<long>(batch, std::min<long>((long)M * D, preferred_batch(n))));
   DevBuf ws(stem_ws_bytes(n, S, A, L, (int)batch, (long)M * D));
-  // more than one batch: the slice loop is captured once and replayed per batch
+  // more than one batch: asked for as a graph (captured from eight full batches on)
   run_stem_impl(j, (int)batch, (long)M * D > batch ? TOTEM_RUN_GRAPH : 0, ws.p, ws.bytes, st);
   std::vector<double> det(det_n);
   HIP_OK(hipMemcpyAsync(det.data(), ddet.p, det_n * sizeof(double), hipMemcpyDeviceToHost, st));

@@ -40,9 +40,12 @@ inline float2 unit_float2(double c, double s) {
 // from the value counting 16 times.  The fused stages multiply at every level of a
 // butterfly, so what the wave's norm sees is a column's mean modulus (near 45 degrees no
 // single pair is on the circle: the nearest are off by -3.4e-8 and +5.0e-8), while each
-// pair's own distance goes into the wave.  Weights of 1 to 32 measured: 1024^2 exit waves
-// of 80 slices 4.5e-6 (1), 3.6e-6 (2), 3.0e-6 (8), 3.1e-6 (16), 3.3e-6 (32), images
-// 3.6e-7, 1.7e-7, 8e-7, 2e-7, 2e-7; unit_float2 lets the norm drift to images of 6.9e-6.
+// pair's own distance goes into the wave.  Exit waves of 80 slices against complex128 by
+// weight, 4 / 8 / 16 / 32: 128^2 2.8e-6, 2.6e-6, 2.5e-6, 2.4e-6; 512^2 2.8, 2.7, 2.7, 2.8;
+// 1024^2 3.3, 3.0, 3.1, 3.3 (4.5 at 1, 3.6 at 2); 1536^2 3.3, 3.3, 3.6, 3.9: flat from 8
+// to 16, where the weight was taken.  The images' error (1e-7 to 4e-6) follows what is
+// left of the norm's drift, which no weight orders; unit_float2 lets it drift to 6.9e-6 at
+// 1024^2.
 inline float2 balanced_float2(double c, double s, double& sum) {
   const float c0 = (float)c, s0 = (float)s;
   float best_c = c0, best_s = s0;
