@@ -69,7 +69,7 @@ rows = rng.uniform(1, 2, (S * each, 14))
 rows[:, 3:] = rows[0, 3:]
 def build():
     engine.build_transmission("l", n, S, np.full(S, float(each)), rows, gx, gy, s2, np.ones_like(s2), 0.7, 1.0, 1 << 40)
-need = 2 * each * (n // 2 + 32) * 8              # the tables of one slice
+need = 2 * each * (n // 2 + 16) * 8              # the tables of one slice
 inputs = 24 * S * each + 3 * 8 * n * n           # terms, s2, AperTrue
 stub.stub_capacity(stub.stub_in_use() + inputs + need + (1 << 20))
 build()

@@ -13,7 +13,7 @@ from totem_amd import optics
 pytestmark = pytest.mark.gpu
 
 N, DX = 1024, 0.08
-COUNTS = (16000, 0, 9000, 21000, 500)        # no corrections: chunks of slices 0-3 and 4; with them, of 0-1, 2 and 3-4
+COUNTS = (16000, 0, 9000, 21000, 3000)       # no corrections: chunks of slices 0-3 and 4; with them, of 0-1, 2, 3 and 4
 
 
 def _slice_v(rows, kind, gx, gy, factors, par):
@@ -34,7 +34,7 @@ def _slice_v(rows, kind, gx, gy, factors, par):
 def test_stack_of_several_chunks(engine, corrected):
     import torch
     print("case chunks corrected=%s" % corrected, flush=True)
-    assert 16 * 544 * sum(COUNTS) > 384 << 20
+    assert 16 * 528 * sum(COUNTS) > 384 << 20
     rng = np.random.default_rng(5)
     gx, gy, s2 = optics.reciprocal_grids(N, DX)
     par, sigma = optics.potential_parameter(N, DX), optics.interaction_sigma(200.0)

@@ -170,10 +170,10 @@ struct PotentialPlan {
 // terms in groups of 16, plus a run's own cost (reduction, form factors per pixel)
 // counted as kFormFactorTerms terms.  A rough model that only has to tell plans of about
 // one class a row from plans of shared classes, which lie far apart.  Builds from rows,
-// rows kept whole / split: erf-weighted rows 256^2 x 10 slices 3.95 / 1.09 ms, 512^2 x 16
-// 39.2 / 8.5, 1024^2 x 8 73 / 6.7, with corrections 512^2 x 8 14.1 / 2.7 (split by the
-// rule); a B of its own per row 256^2 x 10 2.39 / 5.18, 512^2 x 6 3.21 / 6.96 (kept
-// whole); of twelve such builds the rule missed one, a single cell at 256^2 (0.31 / 0.24).
+// rows kept whole / split: erf-weighted rows 256^2 x 10 slices 2.02 / 1.03 ms, 512^2 x 16
+// 27.4 / 8.2, 1024^2 x 8 52.9 / 6.5, with corrections 512^2 x 8 8.7 / 2.6 (split by the
+// rule); a B of its own per row 256^2 x 10 1.56 / 2.57, 512^2 x 6 2.41 / 4.58 (kept
+// whole); the rule took the faster form of all twelve builds timed.
 constexpr long kFormFactorTerms = 32;
 static long plan_cost(const std::vector<std::vector<Term>>& slices, size_t n_classes) {
   std::vector<int> cnt(n_classes, 0);
@@ -421,19 +421,20 @@ struct ScratchUse {
 // Phase tables of a chunk of slices (ex and ey together) up to this size; a slice above
 // it is a chunk of its own. A chunk's last workgroups leave part of the chip idle, so
 // fewer, larger chunks are faster, also beyond the memory-side cache: 80 x 1024^2 slices
-// with corrections 5.6 ms (48 MiB), 4.02 (96), 3.83 (192), 3.66 (384), 3.69 (1024); 30
-// erf-weighted ones of 512^2 2.68, 1.77, 1.66, 1.65, 1.51.
+// with corrections 3.73 ms (96 MiB), 3.62 (192), 3.56 (384), 4.47 (768: more scratch than
+// is kept, allocated anew by each build); 30 erf-weighted ones of 512^2 1.57, 1.55, 1.55,
+// 1.56.
 constexpr size_t kPhaseChunkBytes = 384ull << 20;
 // Slices of a chunk, however few terms they hold: a launch's threads are counted in 32
-// bits, and a 2048^2 slice without frequency pairs takes 2^20 of them.
-constexpr int kChunkSlices = 2048;
+// bits, and a 2048^2 slice without frequency pairs takes 2^23 of them.
+constexpr int kChunkSlices = 256;
 // Form factors are tabulated up to this size.
 constexpr size_t kFormTableBytes = 512ull << 20;
 
 // The stack in chunks of slices, four launches per chunk: phase tables, reciprocal-space
 // accumulation, unnormalised inverse FFT (two passes) with exp(i sigma/1000 V) fused into
 // its column pass (or V copied out when asked).  One slice alone fills the chip only at
-// the largest grids (a 256^2 slice has 25 tiles) and its launches are as long as their
+// the largest grids (a 256^2 slice has 81 tiles) and its launches are as long as their
 // start-up: 20 slices of 256^2 took 20 x 23 us of kernels, in one chunk 85 us.
 // Form factors are tabulated when each class is used by two slices or more
 // on average; with as many classes as runs of terms the table would only move them

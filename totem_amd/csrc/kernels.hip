@@ -4,8 +4,8 @@
 //  * k_pass_cols  -- per slice, along columns: forward column FFT -> x propagator ->
 //                    [annular detectors] -> inverse column FFT   (exit slice: detectors only)
 //  * k_reduce_det -- per finished probe: fixed-order compensated FP64 sum of detector partials
-//  * k_form_table / k_phase / k_accumulate_mfma32 -- projected potential in reciprocal space,
-//                    several slices per launch (structure-factor sums on the matrix cores, 32 x 32
+//  * k_form_table / k_phase / k_accumulate_mfma16 -- projected potential in reciprocal space,
+//                    several slices per launch (structure-factor sums on the matrix cores, 16 x 16
 //                    pixel tiles)
 //  * k_fft_rows / k_fft_cols -- plain batched 2-D FFT passes (potential IFFT, tests)
 //
@@ -844,9 +844,9 @@ __global__ void __launch_bounds__(256) k_form_table(const PotClass* __restrict__
 //
 // Per class the sum over terms is a complex matrix product, A[r][j] = ey_j[r] times
 // B[j][c] = ex_j[c] (the weight w_j already in ex), on the matrix cores in FP32
-// (v_mfma_f32_32x32x2f32, two terms per product): lane l supplies A[l % 32][l / 32] and
-// B[l / 32][l % 32], and accumulator element i of lane l is
-// C[8 (i / 4) + 4 (l / 32) + i % 4][l % 32].  The four real products are kept apart,
+// (v_mfma_f32_16x16x4f32, four terms per product): lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16], and accumulator element i of lane l is C[4 (l / 16) + i][l % 16].  The
+// four real products are kept apart,
 //   P1 = Ar Br,  P2 = Ai Bi,  P3 = Ar Bi,  P4 = Ai Br  (summed over terms),
 // because the weights are real and the grid's frequencies come in pairs
 // (ky[N - r] = -ky[r], kx[N - c] = -kx[c]): then ey_j[N - r] = conj(ey_j[r]) and
@@ -859,196 +859,152 @@ __global__ void __launch_bounds__(256) k_form_table(const PotClass* __restrict__
 // and rows / columns in [1, N/2 - 1] also write their pair N - r: every pixel is
 // written once.  Without it (a grid whose frequencies are not paired) the tiles cover
 // the grid.
-// Four waves share a 32 x 32 tile, each taking every fourth group of 8 terms of a class;
-// their sums meet in LDS, where each thread adds those of four tile positions (elements
-// [4w, 4w + 4) of the wave w) and weights the positions' pixels by the class's FP64 form
-// factor at each of them.  A run of more than 64 terms is summed in two halves: a wave
-// leaves the first half's sums in its own part of the LDS (no barrier) and adds the
-// second's.  FP32 sums of n terms in chains of L are off by about 2.5e-8 sqrt(L / 2), and
-// the halves keep L at n / 8, that of eight waves a tile: V of one class of 400, 1600,
-// 4000, 16000 terms at 256^2 is 2.0e-7, 3.0e-7, 4.2e-7, 7.3e-7 from 64 bits as whole runs
-// in eight waves were, against 2.4e-7, 3.9e-7, 5.7e-7, 1.0e-6 as whole runs in four.
-// Halves cost 1% of an 80 x 1024^2 build and 4% of an erf-weighted 512^2 one, whose runs
-// are 50 to 450 terms; eight waves cost 7% and 9% (one tile per CU, nothing beside its
-// reduction), halves summed in LDS as the runs are 5% and 11%, one 16 x 16 quadrant per
-// wave with all terms (no LDS, twice the operands) 14% and 11%.
-// A 32 x 32 tile reads 512 bytes of phases per term for 4096 multiply-adds, half the
-// operand traffic of a 16 x 16 one, and the next group's phases are in flight during the
-// 16 products of the current one.  Bound by the matrix cores and, behind them, the phases
-// from L2 (about 5 TB/s).  Two tiles per CU (242 VGPRs with tabulated real factors; with
-// complex or evaluated ones 256 and some spills), so one's reduction overlaps the other's
-// products; groups of 8 terms are 5% faster than groups of 4.
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-#ifndef TOTEM_ACC_STEPS
-#define TOTEM_ACC_STEPS 4
-#endif
-#ifndef TOTEM_ACC_MINWAVES
-#define TOTEM_ACC_MINWAVES 2
-#endif
-constexpr int kAccWaves = 4;   // waves sharing a tile
-constexpr int kOneChain = 64;  // runs of more terms are summed in two halves
+// Eight waves share a 16 x 16 tile, each taking every eighth group of 16 terms of a class;
+// the partial products of the waves that hold terms are summed in LDS and each thread
+// weights two pixels by the class's FP64 form factors there, formed or fetched before the
+// sum (formed after it, 64^2 and 128^2 slices of many classes take 6 to 20% longer).  The
+// waves also keep FP32 chains short: a sum in chains of L
+// terms is off by about 2.5e-8 sqrt(L / 2), here L = n / 8 of a run's n (V of one class of
+// 1600 / 16000 terms at 256^2: 3.0e-7 / 7.4e-7; 3.9e-7 / 1.0e-6 with chains of n / 4).
+// Bound by the phases from L2 and the matrix cores where runs are long, by each run's
+// reduction where they are short; 56 VGPRs and 32 KiB let four tiles share a CU.  Tiles of
+// 32 x 32 by four waves (half the operands, but a quarter of the workgroups, eight times the
+// pixels per thread and 242 VGPRs) are slower throughout, us per launch 32 / 16: one slice
+// of 600 terms in 3 classes 68 / 15 at 256^2, 97 / 49 at 1024^2; 16 x 256^2 of 600 48 / 38;
+// 8 x 1024^2 of 4000 980 / 850, and of 120 in 30 classes 542 / 458; whole builds 80 x 1024^2
+// with corrections 3.68 / 3.55 ms, 30 x 512^2 erf-weighted 1.70 / 1.55.
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+constexpr int kAccWaves = 8;  // waves sharing a tile
+// tiles along a side: of [0, np / 2] (paired frequencies) or of [0, np)
+__host__ __device__ constexpr int acc_tiles(int np, bool sym) { return sym ? np / 32 + 1 : np / 16; }
 enum FormMode : int { kFormEval, kFormRe, kFormComplex };
 template <int FORM>
-__global__ void __launch_bounds__(64 * kAccWaves, TOTEM_ACC_MINWAVES)
-k_accumulate_mfma32(const float2* __restrict__ ex, const float2* __restrict__ ey, const PotSlice* __restrict__ slices,
+__global__ void __launch_bounds__(64 * kAccWaves)
+k_accumulate_mfma16(const float2* __restrict__ ex, const float2* __restrict__ ey, const PotSlice* __restrict__ slices,
                     long term_base, const PotSeg* __restrict__ segs, const PotClass* __restrict__ classes,
                     const double* __restrict__ ff_re, const double* __restrict__ ff_im, const double* __restrict__ s2,
                     const double* __restrict__ aper_true, const double* __restrict__ corr, double parameter, int np,
                     int nc, int sym, float2* __restrict__ vshift) {
-  constexpr int W = kAccWaves, U = TOTEM_ACC_STEPS, GT = 2 * U;  // waves; matrix steps, terms per group
-  constexpr int NP = 4, NO = 4 * NP;  // tile positions and pixels per thread
-  static_assert(W == 4, "wave w sums accumulator elements [4w, 4w + 4)");
-  __shared__ float4 red[W][4][4][64];  // [wave][product][elements [4q, 4q + 4)][lane]
-  static_assert(sizeof(red) <= kLdsLimit, "accumulation LDS above 64 KiB");
+  constexpr int W = kAccWaves, NO = 1024 / (64 * W);  // waves; pixels per thread
+  constexpr int U = 4, GT = 4 * U;                      // matrix steps, terms per group
+  static_assert(W == 8, "two pixels per thread");
+  __shared__ float red[W][4][256];  // [wave][product][64 * element + lane]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int dt = nc / 32, tiles = dt * dt;
+  const int half = np / 2;
+  const int dt = acc_tiles(np, sym != 0), tiles = dt * dt;
   const int sl = blockIdx.x / tiles, tile = blockIdx.x - sl * tiles;
   const int tr = tile / dt, tc = tile - tr * dt;
-  const int r0 = tr * 32, c0 = tc * 32;
+  const int r0 = tr * 16, c0 = tc * 16;
+  const int li = lane & 15, lk = lane >> 4;
   const PotSlice ps = slices[sl];
   const size_t np2 = (size_t)np * np;
-  const int half = np / 2;
-  // this thread's positions (accumulator element and lane at which they are summed) and pixels
+  // this thread's tile position, where its sums stand in LDS, and its pixels
+  const int pos = threadIdx.x & 255, pr = pos >> 4, pc = pos & 15;
+  const int src = 64 * (pr & 3) + (pr >> 2) * 16 + pc;
   int pix[NO];  // -1: no such pixel
-  double s2v[FORM == kFormEval ? NO : 1], vr[NO], vi[NO];
+  bool cj_r[NO], cj_c[NO];
+  double s2v[NO], vr[NO], vi[NO];
 #pragma unroll
-  for (int u = 0; u < NP; ++u) {
-    const int r = r0 + 8 * wave + 4 * (lane >> 5) + u, c = c0 + (lane & 31);
-#pragma unroll
-    for (int quad = 0; quad < 4; ++quad) {  // bit 0: column pair, bit 1: row pair
-      const bool cj_c = quad & 1, cj_r = quad >> 1;
-      const int o = 4 * u + quad;
-      const bool ok = sym ? (r <= half && c <= half && (!cj_r || (r >= 1 && r < half)) &&
-                             (!cj_c || (c >= 1 && c < half)))
-                          : quad == 0;
-      pix[o] = ok ? (cj_r ? np - r : r) * np + (cj_c ? np - c : c) : -1;
-      if constexpr (FORM == kFormEval) s2v[o] = ok ? s2[pix[o]] : 0.0;
-      vr[o] = vi[o] = 0.0;
-    }
+  for (int o = 0; o < NO; ++o) {
+    const int quad = (threadIdx.x >> 8) + 2 * o;  // bit 0: column pair, bit 1: row pair
+    const int r = r0 + pr, c = c0 + pc;
+    cj_c[o] = quad & 1;
+    cj_r[o] = quad >> 1;
+    const bool ok = sym ? (r <= half && c <= half && (!cj_r[o] || (r >= 1 && r < half)) &&
+                           (!cj_c[o] || (c >= 1 && c < half)))
+                        : quad == 0;
+    pix[o] = ok ? (cj_r[o] ? np - r : r) * np + (cj_c[o] ? np - c : c) : -1;
+    s2v[o] = FORM == kFormEval && ok ? s2[pix[o]] : 0.0;
+    vr[o] = vi[o] = 0.0;
   }
-  // byte offsets of this lane's phases in a group of terms
-  int oa[U], ob[U];
+  int oa[U], ob[U];  // byte offsets of this lane's phases in a group of terms
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const int row = (2 * u + (lane >> 5)) * nc;
-    oa[u] = (row + r0 + (lane & 31)) * (int)sizeof(float2);
-    ob[u] = (row + c0 + (lane & 31)) * (int)sizeof(float2);
+    const int row = (4 * u + lk) * nc;
+    oa[u] = (row + r0 + li) * (int)sizeof(float2);
+    ob[u] = (row + c0 + li) * (int)sizeof(float2);
   }
-  for (int sgi = ps.seg; sgi < ps.seg + ps.n_seg; ++sgi) {
-    const PotSeg sg = segs[sgi];
+  const int base = (int)(ps.term - term_base);  // within the chunk
+  const int last = ps.seg + ps.n_seg - 1;
+  PotSeg sg, coming;
+  if (ps.n_seg > 0) coming = segs[ps.seg];
+  for (int sgi = ps.seg; sgi <= last; ++sgi) {
+    sg = coming;
+    coming = segs[min(sgi + 1, last)];  // in flight during this run
     if (sg.dup) continue;
-    const int base = (int)(ps.term - term_base);  // within the chunk
-    // phases of the group of terms [j, j + GT) (zero beyond the class's last term)
-    auto load = [&](int j, float2* x, float2* y) {
-      const int left = min(max(sg.end - j, 0), GT);
+    floatx4 p[4] = {};
+    for (int j = sg.begin + GT * wave; j < sg.end; j += GT * W) {
+      const int left = min(sg.end - j, GT);  // the phases of later terms read as zero
       const size_t at = (size_t)(base + j) * nc;
       const auto ra = buf_rsrc(ey + at, (unsigned)(left * nc * (int)sizeof(float2)));
       const auto rb = buf_rsrc(ex + at, (unsigned)(left * nc * (int)sizeof(float2)));
+      float2 a[U], b[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        x[u] = bld(ra, oa[u], 0);
-        y[u] = bld(rb, ob[u], 0);
+        a[u] = bld(ra, oa[u], 0);
+        b[u] = bld(rb, ob[u], 0);
       }
-    };
-    // this wave's groups of terms before `end`, from j on; a and b hold group j
-    floatx16 p[4];
-    float2 a[U], b[U], an[U], bn[U];
-    int j = sg.begin + GT * wave;
-    auto products = [&](int end) {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) p[k] = floatx16{};
-      for (; j < end; j += GT * W) {
-        load(j + GT * W, an, bn);
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          p[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].x, p[0], 0, 0, 0);
-          p[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].y, p[1], 0, 0, 0);
-          p[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].x, b[u].y, p[2], 0, 0, 0);
-          p[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u].y, b[u].x, p[3], 0, 0, 0);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          a[u] = an[u];
-          b[u] = bn[u];
-        }
+      for (int u = 0; u < U; ++u) {
+        p[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].x, p[0], 0, 0, 0);
+        p[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].y, p[1], 0, 0, 0);
+        p[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].y, p[2], 0, 0, 0);
+        p[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].x, p[3], 0, 0, 0);
       }
-    };
-    auto store = [&](bool add) {
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float4& m = red[wave][k][i][lane];
-          float4 v = make_float4(p[k][4 * i], p[k][4 * i + 1], p[k][4 * i + 2], p[k][4 * i + 3]);
-          if (add) {
-            const float4 h = m;
-            v = make_float4(h.x + v.x, h.y + v.y, h.z + v.z, h.w + v.w);
-          }
-          m = v;
-        }
-    };
-    const int len = sg.end - sg.begin;
-    const bool halves = len > kOneChain;
-    load(j, a, b);
-    if (halves) {
-      products(sg.begin + (len + 2 * GT * W - 1) / (2 * GT * W) * (GT * W));
-      store(false);
     }
-    products(sg.end);
     double fr[NO], fi[NO];
     auto factors = [&](int cls) {
 #pragma unroll
       for (int o = 0; o < NO; ++o) {
-        const size_t at = cls * np2 + max(pix[o], 0);
-        fr[o] = ff_re[at];
-        if constexpr (FORM == kFormComplex) fi[o] = ff_im[at];
+        if constexpr (FORM == kFormEval) {
+          const double2 f = pix[o] < 0 ? make_double2(0.0, 0.0)
+                                       : form_factor(classes[cls], s2v[o], corr, pix[o], np2);
+          fr[o] = f.x;
+          fi[o] = f.y;
+        } else {
+          const size_t at = cls * np2 + max(pix[o], 0);
+          fr[o] = ff_re[at];
+          if constexpr (FORM == kFormComplex) fi[o] = ff_im[at];
+        }
       }
     };
-    if constexpr (FORM != kFormEval) factors(sg.cls);
-    store(halves);
+    factors(sg.cls);  // tabulated ones in flight during the sums
+    const int waves = min((sg.end - sg.begin + GT - 1) / GT, W);  // that hold terms of the run
+    if (wave < waves) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[wave][k][64 * i + lane] = p[k][i];
+    }
     __syncthreads();
-    float q[4][NP];
+    float q[4] = {};
+    if (waves == W) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float4 t = red[0][k][wave][lane];
+      for (int w = 0; w < W; ++w)
 #pragma unroll
-      for (int w = 1; w < W; ++w) {
-        const float4 v = red[w][k][wave][lane];
-        t = make_float4(t.x + v.x, t.y + v.y, t.z + v.z, t.w + v.w);
-      }
-      q[k][0] = t.x;
-      q[k][1] = t.y;
-      q[k][2] = t.z;
-      q[k][3] = t.w;
+        for (int k = 0; k < 4; ++k) q[k] += red[w][k][src];
+    } else {
+      for (int w = 0; w < waves; ++w)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) q[k] += red[w][k][src];
     }
     __syncthreads();  // read before the next run's sums are stored
-    for (int run = sgi, cls = sg.cls;;) {  // the run's class and those of its repetitions
+    for (int next = sg.next;;) {  // the run's class and those of its repetitions
 #pragma unroll
-      for (int u = 0; u < NP; ++u)
-#pragma unroll
-        for (int quad = 0; quad < 4; ++quad) {
-          const bool cj_c = quad & 1, cj_r = quad >> 1;
-          const int o = 4 * u + quad;
-          if constexpr (FORM == kFormEval) {
-            if (pix[o] < 0) continue;
-            const double2 f = form_factor(classes[cls], s2v[o], corr, pix[o], np2);
-            fr[o] = f.x;
-            fi[o] = f.y;
-          }
-          const double sre = cj_r == cj_c ? (double)(q[0][u] - q[1][u]) : (double)(q[0][u] + q[1][u]);
-          const double sim = (double)(cj_c ? -q[2][u] : q[2][u]) + (double)(cj_r ? -q[3][u] : q[3][u]);
-          if constexpr (FORM == kFormRe) {
-            vr[o] += fr[o] * sre;
-            vi[o] += fr[o] * sim;
-          } else {
-            vr[o] += fr[o] * sre - fi[o] * sim;
-            vi[o] += fr[o] * sim + fi[o] * sre;
-          }
+      for (int o = 0; o < NO; ++o) {
+        const double sre = cj_r[o] == cj_c[o] ? (double)(q[0] - q[1]) : (double)(q[0] + q[1]);
+        const double sim = (double)(cj_c[o] ? -q[2] : q[2]) + (double)(cj_r[o] ? -q[3] : q[3]);
+        if constexpr (FORM == kFormRe) {
+          vr[o] += fr[o] * sre;
+          vi[o] += fr[o] * sim;
+        } else {
+          vr[o] += fr[o] * sre - fi[o] * sim;
+          vi[o] += fr[o] * sim + fi[o] * sre;
         }
-      run = segs[run].next;
-      if (run < 0) break;
-      cls = segs[run].cls;
-      if constexpr (FORM != kFormEval) factors(cls);
+      }
+      if (next < 0) break;
+      factors(segs[next].cls);
+      next = segs[next].next;
     }
   }
   float2* const out = vshift + sl * np2;
@@ -1406,8 +1362,8 @@ bool hermitian_pairs(const double* kx1, const double* ky1, int np) {
   return true;
 }
 
-// whole 32-entry tiles of [0, np/2] (paired frequencies) or of [0, np)
-int phase_columns(int np, bool sym) { return ((sym ? np / 2 + 1 : np) + 31) / 32 * 32; }
+// whole 16-entry tiles of [0, np/2] (paired frequencies) or of [0, np)
+int phase_columns(int np, bool sym) { return 16 * acc_tiles(np, sym); }
 
 void repeated_runs(hipStream_t st, const PotSlice* slices, int n_slices, PotSeg* segs, const double* tx,
                    const double* ty, const double* wt, unsigned char* dup) {
@@ -1435,18 +1391,18 @@ void accumulate(hipStream_t st, const float2* ex, const float2* ey, const PotSli
                 long term_base, const PotSeg* segs, const PotClass* classes, const double* ff_re, const double* ff_im,
                 const double* s2, const double* aper_true, const double* corr, double parameter, int np, bool sym,
                 float2* vshift) {
-#define X(S) static_assert(S % 32 == 0 && S <= 32768, "potential tiles: whole tiles without pairs, 32-bit pixels");
+#define X(S) static_assert(S % 16 == 0 && S <= 32768, "potential tiles: whole tiles without pairs, 32-bit pixels");
   TOTEM_FOR_SIZES(X)
 #undef X
-  const int nc = phase_columns(np, sym), dt = nc / 32;
-  const dim3 grid((unsigned)(n_slices * dt * dt));
+  const int nc = phase_columns(np, sym), dt = acc_tiles(np, sym);
   auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(64 * kAccWaves), 0, st, ex, ey, slices, term_base, segs, classes, ff_re, ff_im, s2,
-                       aper_true, corr, parameter, np, nc, sym ? 1 : 0, vshift);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(n_slices * dt * dt)), dim3(64 * kAccWaves), 0, st, ex, ey, slices,
+                       term_base, segs, classes, ff_re, ff_im, s2, aper_true, corr, parameter, np, nc, sym ? 1 : 0,
+                       vshift);
   };
-  if (ff_im) launch(k_accumulate_mfma32<kFormComplex>);
-  else if (ff_re) launch(k_accumulate_mfma32<kFormRe>);
-  else launch(k_accumulate_mfma32<kFormEval>);
+  if (ff_im) launch(k_accumulate_mfma16<kFormComplex>);
+  else if (ff_re) launch(k_accumulate_mfma16<kFormRe>);
+  else launch(k_accumulate_mfma16<kFormEval>);
 }
 
 }  // namespace totem

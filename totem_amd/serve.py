@@ -106,7 +106,7 @@ def scratch_bytes(cfg):
     slices (up to 384 MiB, more only for a slice that needs it) and form factors of every class
     (up to 512 MiB).  One build at a time uses it; a scratch above 512 MiB is given back."""
     x = np.asarray(cfg.atoms, dtype=np.float64)
-    term = 16 * (-(-(cfg.np_side // 2 + 1) // 32) * 32)
+    term = 16 * 16 * (cfg.np_side // 32 + 1)                  # x and y phases of whole 16-pixel tiles
     rows = 2 * len(x)                                         # corrections double the rows
     phases = max(min(384 << 20, term * rows), term * (rows // max(cfg.n_slices, 1) + 64))
     if cfg.multiceng:                                         # rows with coefficients of their own near faces
