@@ -425,6 +425,10 @@ struct ScratchUse {
 // is kept, allocated anew by each build); 30 erf-weighted ones of 512^2 1.57, 1.55, 1.55,
 // 1.56.
 constexpr size_t kPhaseChunkBytes = 384ull << 20;
+// A chunk's tables are kept smaller beside large form tables, down to this size, so that
+// the scratch as a whole may stay for the next build (allocated anew it costs 1.2 ms: 80 x
+// 1024^2 erf-weighted at multiceng 0.5, 176 MB of form factors, 31.0 ms).
+constexpr size_t kPhaseChunkMin = 128ull << 20;
 // Slices of a chunk, however few terms they hold: a launch's threads are counted in 32
 // bits, and a 2048^2 slice without frequency pairs takes 2^23 of them.
 constexpr int kChunkSlices = 256;
@@ -443,7 +447,6 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
   const int np = p.np, S = p.S;
   const size_t np2 = (size_t)np * np;
   const size_t term_bytes = 2 * (size_t)phase_columns(np, p.sym) * sizeof(float2);
-  const long per_chunk = std::max<long>(1, (long)(kPhaseChunkBytes / term_bytes));
   ScratchUse use{sc, st};
   std::vector<PotSlice> slices(S);
   for (int s = 0; s < S; ++s)
@@ -466,8 +469,12 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
   upload(sc.slices, slices, st);
   const size_t ff_bytes = (size_t)p.n_classes * np2 * sizeof(double) * (p.absorptive ? 2 : 1);
   bool tabulated = p.seg_off[S] >= 2L * p.n_classes && ff_bytes > 0 && ff_bytes <= kFormTableBytes;
+  // phase tables beside the rest of the scratch within what is kept for the next build
+  const size_t rest = (tabulated ? ff_bytes : 0) + S * sizeof(PotSlice) + p.term_off[S];
+  const size_t chunk_bytes =
+      std::min(kPhaseChunkBytes, std::max(kPhaseChunkMin, kKeepBuilderScratch - std::min(kKeepBuilderScratch, rest)));
   try {
-    reserve_tables(per_chunk, tabulated ? ff_bytes : 0);
+    reserve_tables(std::max<long>(1, (long)(chunk_bytes / term_bytes)), tabulated ? ff_bytes : 0);
   } catch (const Error& e) {
     // a nearly full device: one slice at a time, form factors formed in each, as much
     // scratch as the largest slice needs

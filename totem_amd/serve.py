@@ -102,17 +102,21 @@ def footprint_bytes(cfg, M=None, A=None):
 
 
 def scratch_bytes(cfg):
-    """Bound of the potential builder's scratch for a request's build: phase tables of a chunk of
-    slices (up to 384 MiB, more only for a slice that needs it) and form factors of every class
-    (up to 512 MiB).  One build at a time uses it; a scratch above 512 MiB is given back."""
+    """Bound of the potential builder's scratch for a request's build: form factors of every class
+    (up to 512 MiB) and phase tables of a chunk of slices (384 MiB, less beside large form tables
+    down to 128 MiB, more only for a slice that needs it).  One build at a time uses it; a scratch
+    above 512 MiB is given back."""
     x = np.asarray(cfg.atoms, dtype=np.float64)
     term = 16 * 16 * (cfg.np_side // 32 + 1)                  # x and y phases of whole 16-pixel tiles
     rows = 2 * len(x)                                         # corrections double the rows
-    phases = max(min(384 << 20, term * rows), term * (rows // max(cfg.n_slices, 1) + 64))
     if cfg.multiceng:                                         # rows with coefficients of their own near faces
-        return int(phases) + (512 << 20)
-    classes = 2 * len(np.unique(x[:, [0, 4, 5, 6]], axis=0)) if len(x) else 0
-    return int(phases + min(512 << 20, 8 * classes * cfg.np_side ** 2))
+        form, rows = 512 << 20, 15 * rows
+    else:
+        classes = 2 * len(np.unique(x[:, [0, 4, 5, 6]], axis=0)) if len(x) else 0
+        form = min(512 << 20, 8 * classes * cfg.np_side ** 2)
+    chunk = min(384 << 20, term * rows) if form <= 128 << 20 else min(term * rows, max(128 << 20, (512 << 20) - form))
+    slice_rows = rows // max(cfg.n_slices, 1) + 64
+    return int(form + max(chunk, term * slice_rows))
 
 
 class Admission:
