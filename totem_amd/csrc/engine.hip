@@ -439,7 +439,7 @@ constexpr size_t kFormTableBytes = 512ull << 20;
 // accumulation, unnormalised inverse FFT (two passes) with exp(i sigma/1000 V) fused into
 // its column pass (or V copied out when asked).  One slice alone fills the chip only at
 // the largest grids (a 256^2 slice has 81 tiles) and its launches are as long as their
-// start-up: 20 slices of 256^2 took 20 x 23 us of kernels, in one chunk 85 us.
+// start-up: 20 slices of 256^2 took 20 x 23 us of kernels, in one chunk 43 us.
 // Form factors are tabulated when each class is used by two slices or more
 // on average; with as many classes as runs of terms the table would only move them
 // through memory.

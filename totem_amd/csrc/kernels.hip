@@ -865,14 +865,16 @@ __global__ void __launch_bounds__(256) k_form_table(const PotClass* __restrict__
 // sum (formed after it, 64^2 and 128^2 slices of many classes take 6 to 20% longer).  The
 // waves also keep FP32 chains short: a sum in chains of L
 // terms is off by about 2.5e-8 sqrt(L / 2), here L = n / 8 of a run's n (V of one class of
-// 1600 / 16000 terms at 256^2: 3.0e-7 / 7.4e-7; 3.9e-7 / 1.0e-6 with chains of n / 4).
+// 1600 / 16000 terms at 256^2: 3.0e-7 / 7.4e-7; 3.9e-7 / 1.0e-6 with chains of n / 4).  Runs
+// of up to 64 terms go in groups of 8, for the same reason (16 terms 1.68e-7 -> 1.62e-7),
+// and a group of 8 or fewer skips its other half's products.
 // Bound by the phases from L2 and the matrix cores where runs are long, by each run's
 // reduction where they are short; 56 VGPRs and 32 KiB let four tiles share a CU.  Tiles of
 // 32 x 32 by four waves (half the operands, but a quarter of the workgroups, eight times the
 // pixels per thread and 242 VGPRs) are slower throughout, us per launch 32 / 16: one slice
 // of 600 terms in 3 classes 68 / 15 at 256^2, 97 / 49 at 1024^2; 16 x 256^2 of 600 48 / 38;
 // 8 x 1024^2 of 4000 980 / 850, and of 120 in 30 classes 542 / 458; whole builds 80 x 1024^2
-// with corrections 3.68 / 3.55 ms, 30 x 512^2 erf-weighted 1.70 / 1.55.
+// with corrections 3.68 / 3.54 ms, 30 x 512^2 erf-weighted 1.70 / 1.52.
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int kAccWaves = 8;  // waves sharing a tile
 // tiles along a side: of [0, np / 2] (paired frequencies) or of [0, np)
@@ -933,23 +935,37 @@ k_accumulate_mfma16(const float2* __restrict__ ex, const float2* __restrict__ ey
     coming = segs[min(sgi + 1, last)];  // in flight during this run
     if (sg.dup) continue;
     floatx4 p[4] = {};
-    for (int j = sg.begin + GT * wave; j < sg.end; j += GT * W) {
-      const int left = min(sg.end - j, GT);  // the phases of later terms read as zero
+    const int gt = sg.end - sg.begin <= 8 * W ? 8 : GT;  // short runs: half groups, on more waves
+    for (int j = sg.begin + gt * wave; j < sg.end; j += gt * W) {
+      const int left = min(sg.end - j, gt);  // the phases of later terms read as zero
       const size_t at = (size_t)(base + j) * nc;
       const auto ra = buf_rsrc(ey + at, (unsigned)(left * nc * (int)sizeof(float2)));
       const auto rb = buf_rsrc(ex + at, (unsigned)(left * nc * (int)sizeof(float2)));
       float2 a[U], b[U];
+      auto load = [&](int u0) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        a[u] = bld(ra, oa[u], 0);
-        b[u] = bld(rb, ob[u], 0);
-      }
+        for (int u = u0; u < u0 + U / 2; ++u) {
+          a[u] = bld(ra, oa[u], 0);
+          b[u] = bld(rb, ob[u], 0);
+        }
+      };
+      auto products = [&](int u0) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        p[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].x, p[0], 0, 0, 0);
-        p[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].y, p[1], 0, 0, 0);
-        p[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].y, p[2], 0, 0, 0);
-        p[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].x, p[3], 0, 0, 0);
+        for (int u = u0; u < u0 + U / 2; ++u) {
+          p[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].x, p[0], 0, 0, 0);
+          p[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].y, p[1], 0, 0, 0);
+          p[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].y, p[2], 0, 0, 0);
+          p[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].x, p[3], 0, 0, 0);
+        }
+      };
+      if (left > GT / 2) {
+        load(0);
+        load(U / 2);
+        products(0);
+        products(U / 2);
+      } else {  // the other half holds zeros
+        load(0);
+        products(0);
       }
     }
     double fr[NO], fi[NO];
@@ -969,7 +985,7 @@ k_accumulate_mfma16(const float2* __restrict__ ex, const float2* __restrict__ ey
       }
     };
     factors(sg.cls);  // tabulated ones in flight during the sums
-    const int waves = min((sg.end - sg.begin + GT - 1) / GT, W);  // that hold terms of the run
+    const int waves = min((sg.end - sg.begin + gt - 1) / gt, W);  // that hold terms of the run
     if (wave < waves) {
 #pragma unroll
       for (int k = 0; k < 4; ++k)
