@@ -19,7 +19,7 @@ for name in ("in_use", "peak", "in_use_at_info"):
 stub.stub_capacity.argtypes = [ctypes.c_size_t]
 stub.stub_fill.argtypes = [ctypes.c_size_t, ctypes.c_int]
 stub.stub_fail_copy.argtypes = [ctypes.c_long]
-for name in ("launches", "pending"):
+for name in ("launches", "pending", "events"):
     getattr(stub, "stub_" + name).restype = ctypes.c_long
 stub.stub_widest.restype = ctypes.c_ulonglong
 stub.stub_reset_peak.restype = None

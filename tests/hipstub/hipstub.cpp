@@ -27,7 +27,7 @@ size_t capacity = (size_t)288 << 30, in_use = 0, peak = 0, in_use_at_info = 0;
 size_t fill_bytes = 0;
 int fill_value = 0;
 long copies_to_fail = -1;      // copies to the host until one fails
-long launches = 0;
+long launches = 0, events = 0;
 unsigned long long widest = 0;  // threads of the widest launch along x
 hipError_t last = hipSuccess;
 std::map<const void*, void*> symbols;
@@ -60,6 +60,7 @@ size_t stub_peak() { return peak; }
 void stub_reset_peak() { peak = in_use; }
 size_t stub_in_use_at_info() { return in_use_at_info; }
 long stub_launches() { return launches; }
+long stub_events() { return events; }
 unsigned long long stub_widest() { return widest; }
 long stub_pending() {
   long n = 0;
@@ -167,6 +168,7 @@ hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t* e) {
+  ++events;
   *e = reinterpret_cast<hipEvent_t>(handle<char>());
   return hipSuccess;
 }

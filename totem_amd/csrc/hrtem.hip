@@ -253,6 +253,8 @@ __global__ void __launch_bounds__(256) k_tcc_field(const double2* __restrict__ w
 // kernels and the inputs' upload are left outside it (3.85 -> 3.35 ms a call). A chunk
 // holds this many bytes of images (4 MiB: 4.03 ms, 64 MiB: 3.50 ms).
 constexpr size_t kImageChunkBytes = 16ull << 20;
+// Chunks of a batch at most (larger ones then): their events are kept.
+constexpr int kImageChunks = 64;
 
 // The stream images leave on and a chunk's events, per device; made at the first batch of
 // several chunks and kept (making them takes 0.4 ms), used under the scratch's lock.
@@ -375,7 +377,7 @@ void hrtem_images_impl(const totem_hrtem_desc& d, double* paras_out, double* ima
                      sc.ai.as<double>(), B, sc.paras.as<double>());
   if (paras_out)
     HIP_OK(hipMemcpyAsync(paras_out, sc.paras.p, (size_t)B * kPara * sizeof(double), hipMemcpyDeviceToHost, st));
-  const int per = (int)std::max<size_t>(1, kImageChunkBytes / (NN * sizeof(double)));
+  const int per = std::max({1, (int)(kImageChunkBytes / (NN * sizeof(double))), (B + kImageChunks - 1) / kImageChunks});
   const int chunks = (B + per - 1) / per;
   auto form = [&](int b0, int cnt) {
     const long total = (long)cnt * (long)NN;
