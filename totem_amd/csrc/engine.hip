@@ -447,8 +447,8 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
   const int np = p.np, S = p.S;
   const size_t np2 = (size_t)np * np;
   const size_t term_bytes = 2 * (size_t)phase_columns(np, p.sym) * sizeof(float2);
-  ScratchUse use{sc, st};
   std::vector<PotSlice> slices(S);
+  ScratchUse use{sc, st};  // ends before the slice list it may be copying
   for (int s = 0; s < S; ++s)
     slices[s] = {p.term_off[s], (int)p.seg_off[s], (int)(p.seg_off[s + 1] - p.seg_off[s])};
   std::vector<int> chunks;  // chunk boundaries

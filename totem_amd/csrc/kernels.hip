@@ -863,11 +863,11 @@ __global__ void __launch_bounds__(256) k_form_table(const PotClass* __restrict__
 // the partial products of the waves that hold terms are summed in LDS and each thread
 // weights two pixels by the class's FP64 form factors there, formed or fetched before the
 // sum (formed after it, 64^2 and 128^2 slices of many classes take 6 to 20% longer).  The
-// waves also keep FP32 chains short: a sum in chains of L
-// terms is off by about 2.5e-8 sqrt(L / 2), here L = n / 8 of a run's n (V of one class of
-// 1600 / 16000 terms at 256^2: 3.0e-7 / 7.4e-7; 3.9e-7 / 1.0e-6 with chains of n / 4).  Runs
-// of up to 64 terms go in groups of 8, for the same reason (16 terms 1.68e-7 -> 1.62e-7),
-// and a group of 8 or fewer skips its other half's products.
+// waves also keep FP32 chains short: a sum in chains of L terms is off by about
+// 2.5e-8 sqrt(L / 2), here L = n / 8 of a run's n (V of one class of 1600 / 16000 terms at
+// 256^2: 3.0e-7 / 7.4e-7; 3.9e-7 / 1.0e-6 with chains of n / 4).  Runs of up to 64 terms go
+// in groups of 8 for the same reason (16 terms 1.68e-7 -> 1.63e-7), and a group of 8 or
+// fewer skips its other half's products.
 // Bound by the phases from L2 and the matrix cores where runs are long, by each run's
 // reduction where they are short; 56 VGPRs and 32 KiB let four tiles share a CU.  Tiles of
 // 32 x 32 by four waves (half the operands, but a quarter of the workgroups, eight times the
