@@ -412,8 +412,9 @@ struct PotScratch {
 struct ScratchUse {
   PotScratch& sc;
   hipStream_t st;
+  bool waited = false;  // the build has waited for the stream itself
   ~ScratchUse() {
-    (void)hipStreamSynchronize(st);
+    if (!waited) (void)hipStreamSynchronize(st);
     if (sc.bytes() > kKeepBuilderScratch) sc.release();
   }
 };
@@ -525,6 +526,7 @@ void potential_run(const PotDev& p, float2* t_dev, double* v_re, double* v_im, h
     HIP_OK(hipGetLastError());
   }
   HIP_OK(hipStreamSynchronize(st));
+  use.waited = true;
 }
 
 // Flattens a plan's terms slice by slice, stably grouped by class within a slice.
